@@ -361,6 +361,14 @@ int mw8_moe_gemm_act_w8a8_bf16(const int8_t* A, const float* sa, const int8_t* W
                                int32_t top_k, int64_t num_valid, int64_t N, int64_t K, int32_t E,
                                int32_t block_size, int32_t act, void* out, mw8_stream_t stream);
 
+/*
+ * Whether mw8_moe_gemm_act_w8a8_bf16 is the faster first step of a prefill
+ * MoE layer of these sizes (64/128-row blocks), against
+ * mw8_moe_gemm_w8a8_bf16 and a separate activation (host only; follows the
+ * grouped configuration override; no reference counterpart).
+ */
+int32_t mw8_moe_gemm_act_preferred(int64_t num_valid, int64_t N, int64_t K, int32_t E);
+
 /* Same, raw int32 accumulators out [num_valid, N] (parity hook; no reference counterpart). */
 int mw8_moe_gemm_w8a8_i32(const int8_t* A, const int8_t* W, const int32_t* sorted_ids,
                           const int32_t* expert_ids, const int32_t* num_post_pad,

@@ -61,6 +61,7 @@ int moe_gemm_sum_w8a8(const int8_t*, const float*, const int8_t*, const float*, 
                       const int32_t*, const int32_t*, int64_t, const float*, int, int64_t, int64_t,
                       int64_t, int, void*, hipStream_t);
 int moe_gemm_sum_lds_bytes(int64_t, int64_t, int);
+int moe_gemm_act_preferred(int64_t, int64_t, int64_t, int);
 int moe_gemm_topk_w8a8(const int8_t*, const float*, const int8_t*, const float*, const int32_t*, const float*, int,
                        int64_t, int64_t, int64_t, int, void*, int, hipStream_t);
 int moe_gemm_sum_topk_w8a8(const int8_t*, const float*, const int8_t*, const float*, const int32_t*, const float*,
@@ -224,6 +225,10 @@ int mw8_moe_gemm_sum_topk_w8a8_bf16(const int8_t* A, const float* sa, const int8
                                     mw8_stream_t stream) {
   MW8_ENTRY(mw8::moe_gemm_sum_topk_w8a8(A, sa, W, sw, topk_ids, topk_w, top_k, num_valid, N, K, E, out,
                                         S(stream)));
+}
+
+int32_t mw8_moe_gemm_act_preferred(int64_t num_valid, int64_t N, int64_t K, int32_t E) {
+  return mw8::moe_gemm_act_preferred(num_valid, N, K, E);
 }
 
 int32_t mw8_moe_gemm_sum_supported(int64_t max_sorted, int64_t num_valid, int32_t E) {

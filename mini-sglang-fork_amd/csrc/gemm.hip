@@ -7,6 +7,7 @@
 #include "gemm_kernels.h"
 #include "gemm_ksplit.h"
 #include "gemm_stream.h"
+#include "gemm_walk.h"
 
 namespace mw8 {
 
@@ -324,7 +325,7 @@ constexpr TileCfg kTileCfgs[] = {
     {256, 320, true, 128, 1, false, "tile3_gemm_kernel<256, 320, 128, 2, 4, 2>"},
     // 7: the pipelined persistent walk over 256x256 tiles (bf16 output, at
     // least 6 K stages and one tile per CU; else as cfg 2)
-    {256, 256, true, 128, 1, false, "stream_gemm_kernel<256, 0, false, -1>"},
+    {256, 256, true, 128, 1, false, "stream_gemm_kernel<256>"},
 };
 constexpr int kNumRingCfgs = sizeof(kTileCfgs) / sizeof(kTileCfgs[0]);
 
@@ -566,10 +567,9 @@ int launch_split_reduce(const GemmArgs& g, const SplitPlan& sp, hipStream_t st) 
 }
 
 // The stream walk (gemm_stream.h) over 256 x 256 tiles: one block per CU.
-template <bool kGrouped, int kAct = -1>
 int launch_stream(const GemmArgs& g, unsigned blocks, hipStream_t st) {
-  constexpr int kLds = stream_lds_bytes<256, kAct>();
-  constexpr auto kern = stream_gemm_kernel<256, kEpiBf16, kGrouped, kAct>;
+  constexpr int kLds = stream_lds_bytes<256>();
+  constexpr auto kern = stream_gemm_kernel<256>;
   if (const int rc = set_lds_limit<kern>(kLds)) return rc;
   hipLaunchKernelGGL(kern, dim3(blocks), dim3(512), kLds, st, g);
   return kOk;
@@ -578,9 +578,9 @@ int launch_stream(const GemmArgs& g, unsigned blocks, hipStream_t st) {
 // Whether the stream walk takes a bf16 GEMM: whole 128-byte K stages, at
 // least kStreamMinStages of them, 16-byte output rows, and an output the
 // 32-bit buffer offsets reach.
-bool stream_fits(const GemmArgs& g, int64_t out_rows, int64_t out_cols) {
-  return g.staged_out && g.K % kStreamBK == 0 && g.K / kStreamBK >= kStreamMinStages && out_cols % 8 == 0 &&
-         out_rows * g.ldo * 2 < (int64_t{1} << 31);
+bool stream_fits(const GemmArgs& g) {
+  return g.staged_out && g.K % kStreamBK == 0 && g.K / kStreamBK >= kStreamMinStages && g.N % 8 == 0 &&
+         g.M * g.ldo * 2 < (int64_t{1} << 31);
 }
 
 template <int EPI>
@@ -628,8 +628,8 @@ int dispatch_tile(GemmArgs g, void* ws, size_t ws_bytes, hipStream_t st) {
     case 6: rc = launch_tile3<256, 320, 128, 2, 4, 2, EPI, DenseRows>(g, dim3(tiles), st); break;
     default: {
       const int64_t cus = device_cus();
-      if (EPI == kEpiBf16 && tiles >= cus && stream_fits(g, g.M, g.N))
-        rc = launch_stream<false>(g, static_cast<unsigned>(cus), st);
+      if (EPI == kEpiBf16 && tiles >= cus && stream_fits(g))
+        rc = launch_stream(g, static_cast<unsigned>(cus), st);
       else
         rc = launch_tile3<256, 256, 128, 2, 4, 2, EPI, DenseRows, 0, kLead256>(g, dim3(tiles), st);
       break;
@@ -920,18 +920,49 @@ int launch_grouped_persist(const GemmArgs& g, hipStream_t st) {
   return kOk;
 }
 
+// The grouped walk (gemm_walk.h): one block per CU.  It takes whole 128-byte
+// K stages, at least kWalkMinStages of them, whole 256-row weight tiles, and
+// weights, scales and outputs that 32-bit buffer offsets reach.
+bool walk_takes(int64_t N, int64_t K, int64_t E, int64_t num_valid, int64_t out_cols) {
+  constexpr int64_t kMax = int64_t{1} << 31;
+  return K % kWalkBK == 0 && K / kWalkBK >= kWalkMinStages && N % kWalkBN == 0 && E < kPersistMaxSlots &&
+         num_valid * out_cols * 2 < kMax && N * K < kMax && E * N * 4 < kMax;
+}
+bool walk_fits(const GemmArgs& g) {
+  return g.staged_out && walk_takes(g.N, g.K, g.num_experts, g.num_valid, g.ldo);
+}
+
+template <int kAct>
+int launch_walk(const GemmArgs& g, hipStream_t st) {
+  constexpr auto kern = walk_gemm_kernel<kAct>;
+  if (const int rc = set_lds_limit<kern>(kWalkLds)) return rc;
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(device_cus())), dim3(512), kWalkLds, st, g);
+  return kOk;
+}
+
 // Grouped configurations for 64/128-row alignment blocks (mw8_set_tuning
 // moe_cfg): 0 one 128-wide ring tile per alignment block (tile height =
 // block size), 1 the persistent walk over (expert, column tile, chunk)
 // items with 128x256 tiles on 64-byte K stages, two blocks per CU.
 //
-// Automatic choice, measured on MI355X at config 3 (E 128, top-8, H 2048,
-// I 768; whole layer): with at least 32 pairs per expert on average the
-// persistent chunk walk (cfg 1): 1024 tokens 237 -> 215 us, 4096 tokens
-// 536 -> 459 us against cfg 0; at 16 pairs per expert (256 tokens) cfg 0
-// (167 us against 177).
+// 2 the walk over tall items (gemm_walk.h), which takes whole 128-byte K
+// stages and whole column tiles (walk_fits; else the automatic choice of 0
+// and 1).
+//
+// Automatic choice: the walk wherever it fits and the output is bf16.
+// Measured on MI355X (weights from HBM, us per launch, best of 0 and 1 ->
+// walk; GEMM1 with the activation in its epilogue / GEMM2): E 128, top-8,
+// H 2048, I 768 at 300 / 1024 / 2048 / 4096 / 8192 tokens GEMM1 79 / 85 /
+// 118 / 186 / 300 -> 67 / 72 / 80 / 146 / 236, GEMM2 45 / 59 / 86 / 129 /
+// 218 -> 43 / 52 / 65 / 114 / 193; E 64, top-6, H 4096, I 1152 at 4096
+// tokens 333 / 219 -> 250 / 188; E 16, top-2, H 4096, I 1408 at 2500 tokens
+// 106 / 51 -> 81 / 46.  Where it does not fit: with at least 32 pairs per
+// expert on average the persistent chunk walk (cfg 1): 1024 tokens 237 ->
+// 215 us per layer, 4096 tokens 536 -> 459 us against cfg 0; at 16 pairs per
+// expert (256 tokens) cfg 0 (167 us against 177).
 constexpr int kNumMoeCfgs = 3;
-int default_moe_cfg(const GemmArgs& g) {
+int default_moe_cfg(const GemmArgs& g, int epi) {
+  if (epi == kEpiBf16 && walk_fits(g)) return 2;
   if (g.K % 64 == 0 && g.num_experts < kPersistMaxSlots &&
       g.num_valid >= 32 * static_cast<int64_t>(g.num_experts))
     return 1;
@@ -946,12 +977,10 @@ int launch_grouped_epi(const GemmArgs& g, unsigned blocks, int bm, hipStream_t s
     return launch_tile<128, 128, 128, 2, 2, EPI, SortedRows>(g, grid, st);
   }
   int cfg = g_moe_cfg;
-  if (cfg < 0 || cfg >= kNumMoeCfgs) cfg = default_moe_cfg(g);
+  if (cfg < 0 || cfg >= kNumMoeCfgs) cfg = default_moe_cfg(g, EPI);
   if (cfg == 1 && g.num_experts < kPersistMaxSlots)
     return launch_grouped_persist<128, 256, 64, 2, 2, 3, EPI, 2>(g, st);
-  if (cfg == 2 && EPI == kEpiBf16 && g.num_experts < kPersistMaxSlots && 256 % g.align_bsz == 0 &&
-      stream_fits(g, g.num_valid, g.N))
-    return launch_stream<true>(g, static_cast<unsigned>(device_cus()), st);
+  if (cfg == 2 && EPI == kEpiBf16 && walk_fits(g)) return launch_walk<-1>(g, st);
   if (bm == 64) return launch_grouped3<64, 128, 64, 2, 2, 4, EPI>(g, blocks, st);
   return launch_grouped3<128, 128, 64, 2, 2, 4, EPI>(g, blocks, st);
 }
@@ -1082,16 +1111,25 @@ int launch_moe_gemm_sum(const GemmArgs& g, int64_t max_sorted, hipStream_t st, b
   return kOk;
 }
 
-// Gate|up GEMM with the gated activation fused (persistent chunk walk, the
-// moe cfg 1 tiling): out [rows, N/2] = act(gate) * up, bf16.
+// Gate|up GEMM with the gated activation fused (the grouped walk, or the
+// persistent chunk walk where it does not fit or moe cfg 0 or 1 is forced):
+// out [rows, N/2] = act(gate) * up, bf16.
 int launch_grouped_act(const GemmArgs& g, int act, hipStream_t st) {
   const int cfg = g_moe_cfg;
-  if (cfg == 2 && 256 % g.align_bsz == 0 && stream_fits(g, g.num_valid, g.N / 2)) {
-    if (act == 0) return launch_stream<true, 0>(g, static_cast<unsigned>(device_cus()), st);
-    return launch_stream<true, 1>(g, static_cast<unsigned>(device_cus()), st);
-  }
+  if ((cfg < 0 || cfg >= 2) && walk_fits(g)) return act == 0 ? launch_walk<0>(g, st) : launch_walk<1>(g, st);
   if (act == 0) return launch_grouped_persist<128, 256, 64, 2, 2, 3, kEpiBf16, 2, 0>(g, st);
   return launch_grouped_persist<128, 256, 64, 2, 2, 3, kEpiBf16, 2, 1>(g, st);
+}
+
+// Whether the fused-activation GEMM1 is the faster first step of a prefill
+// MoE layer (64/128-row alignment blocks; w1 [E, N = 2I, K]): wherever the
+// grouped walk takes it (300 tokens at E 128, top-8, H 2048, I 768: 79 us and
+// a 5.6 us activation kernel -> 67 us and a 4 us quantizer), else from 32
+// pairs per expert (the persistent chunk walk's range).
+int moe_gemm_act_preferred(int64_t num_valid, int64_t N, int64_t K, int E) {
+  if (num_valid < 0 || N <= 0 || N % 16 != 0 || K <= 0 || K % 64 != 0 || E < 1 || E >= kPersistMaxSlots) return 0;
+  if ((g_moe_cfg < 0 || g_moe_cfg >= 2) && walk_takes(N, K, E, num_valid, N / 2)) return 1;
+  return num_valid >= 32 * static_cast<int64_t>(E) ? 1 : 0;
 }
 
 }  // namespace mw8

@@ -18,7 +18,8 @@
 //   grouped_persist_kernel -- the same ring walking (expert chunk, column
 //                  tile) items of the fused-MoE GEMM.
 //   (gemm_ksplit.h: in-block split-K tiles for 33-768 rows; gemm_stream.h:
-//   the pipelined persistent walk over 256x256 tiles.)
+//   the pipelined persistent walk over 256x256 tiles; gemm_walk.h: the
+//   grouped walk of the fused-MoE prefill.)
 //   decode_gemm_kernel / decode3_gemm_kernel -- dense small M (decode):
 //                  weight streaming with v_mfma_i32_16x16x64_i8, weight rows
 //                  as the MFMA "A" operand, up to 64 tokens as the "B"

@@ -544,6 +544,12 @@ def fused_moe_kernel_w8a8(
     )
 
 
+def moe_gemm_act_preferred(num_valid_tokens: int, N: int, K: int, num_experts: int) -> bool:
+    """Whether fused_moe_kernel_act_w8a8 is the faster GEMM1 of a prefill
+    layer of these sizes (host only)."""
+    return bool(load().mw8_moe_gemm_act_preferred(num_valid_tokens, N, K, num_experts))
+
+
 def fused_moe_kernel_act_w8a8(
     A: torch.Tensor,
     A_scale: torch.Tensor,
@@ -734,6 +740,7 @@ def moe_sum_reduce(input: torch.Tensor, output: torch.Tensor) -> None:
 
 __all__ = [
     "moe_gemm_sum_supported",
+    "moe_gemm_act_preferred",
     "fused_moe_kernel_sum_w8a8",
     "fused_moe_kernel_topk_w8a8",
     "fused_moe_kernel_sum_topk_w8a8",

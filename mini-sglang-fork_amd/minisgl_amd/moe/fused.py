@@ -48,6 +48,7 @@ from ..kernel import (
     fused_moe_kernel_topk_w8a8,
     fused_moe_kernel_w8a8,
     moe_align_block_size,
+    moe_gemm_act_preferred,
     moe_gemm_sum_supported,
     moe_prepare_small,
     moe_route_quant,
@@ -202,7 +203,7 @@ def _experts_from_routing(
     num_post_pad, k, bsz, activation, apply_router_weight_on_input,
 ) -> torch.Tensor:
     """Steps 4-7: GEMM1, activation + requant, GEMM2, slot sum in place.
-    Prefill batches (>= 32 pairs per expert, 64/128-row blocks) run the
+    Prefill batches (64/128-row blocks, moe_gemm_act_preferred) run the
     activation in GEMM1's epilogue, writing [M*k, I] instead of [M*k, 2I];
     decode batches (16-row blocks) run the slot sum inside GEMM2, which
     writes hidden_states directly; the values are the same bit for bit."""
@@ -222,7 +223,7 @@ def _experts_from_routing(
         return hidden_states
     # one buffer backs both bf16 caches, as in the reference (:157-172)
     cache = torch.empty(M * k * max(N, H), dtype=torch.bfloat16, device=hidden_states.device)
-    if bsz in (64, 128) and M * k >= 32 * E and N % 16 == 0 and K % 64 == 0 and E < 512:
+    if bsz in (64, 128) and moe_gemm_act_preferred(M * k, N, K, E):
         act = cache[: M * k * (N // 2)].view(M * k, N // 2)
         fused_moe_kernel_act_w8a8(
             q_h, s_h, w1, w1_scale, act, sorted_ids, expert_ids, num_post_pad, k, bsz, M * k,

@@ -1,0 +1,107 @@
+"""The grouped walk (moe cfg 2) where it can go wrong: chunk heights around
+the 16-row fragments, the 128-row DMA variant and the 192-row chunk limit,
+empty experts, the fewest K stages, more items than blocks (the ring runs on
+across items), and the fused activation.  Bit-exact against the oracle's
+grouped GEMM; the fused activation bit-identical to the GEMM followed by the
+activation kernel."""
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import announce, bf16_bits_equal
+from minisgl_amd.kernel import (
+    act_and_mul_quant,
+    fused_moe_kernel_act_w8a8,
+    fused_moe_kernel_w8a8,
+    moe_align_block_size,
+    moe_gemm_act_preferred,
+    quant_per_token,
+)
+from minisgl_amd.kernel import lib as mw8lib
+from oracle import w8a8 as orc
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+# pairs per expert: fragment, DMA-variant and chunk edges, none, several chunks
+COUNTS = [1, 15, 16, 17, 0, 64, 65, 127, 128, 129, 175, 191, 192, 193, 0, 256, 257, 320, 383, 384, 385, 31, 33, 0]
+
+
+def _case(counts, k, N, K, seed):
+    """Hand-made routing: pair p of the flat [M, k] ids goes to the expert
+    that a shuffled list of the counts gives it."""
+    gen = torch.Generator().manual_seed(seed)
+    flat = torch.cat([torch.full((c,), e, dtype=torch.int32) for e, c in enumerate(counts)])
+    flat = flat[torch.randperm(flat.numel(), generator=gen)]
+    pad = -flat.numel() % k
+    flat = torch.cat([flat, flat[:pad]])
+    ids = flat.view(-1, k).contiguous()
+    E = len(counts)
+    W = torch.randint(-127, 128, (E, N, K), generator=gen, dtype=torch.int8)
+    SW = torch.rand(E, N, generator=gen) * 1e-2 + 1e-4
+    tw = torch.rand(ids.shape, generator=gen)
+    return ids, W, SW, tw, gen
+
+
+@pytest.mark.parametrize("B", [64, 128])
+@pytest.mark.parametrize("N,K", [(256, 640), (4096, 640), (512, 1152)])
+def test_walk_equals_oracle(N, K, B):
+    k = 2
+    ids, W, SW, tw, gen = _case(COUNTS, k, N, K, N + K)
+    M, E = ids.shape[0], W.shape[0]
+    idsd, twd, Wd, SWd = ids.to(DEV), tw.to(DEV), W.to(DEV), SW.to(DEV)
+    sorted_ids, expert_ids, npp = moe_align_block_size(idsd, B, E)
+    lib = mw8lib.load()
+    try:
+        lib.mw8_set_tuning(-1, -1, 2)
+        for which in (1, 2):
+            announce(f"walk N={N} K={K} B={B} gemm{which}")
+            rows = M if which == 1 else M * k
+            q, s = quant_per_token(torch.randn(rows, K, generator=gen).to(torch.bfloat16).to(DEV))
+            top_k, routed = (k, None) if which == 1 else (1, tw.numpy())
+            y_ref = orc.grouped_gemm_w8a8(q.cpu().numpy(), s.cpu().numpy(), W.numpy(), SW.numpy(), ids.numpy(), top_k,
+                                          routed=routed)
+            out = torch.empty(M * k, N, dtype=torch.bfloat16, device=DEV)
+            for _ in range(2):
+                out.zero_()
+                fused_moe_kernel_w8a8(q, s, Wd, SWd, out, twd, sorted_ids, expert_ids, npp, routed is not None, top_k,
+                                      B, M * k)
+                torch.cuda.synchronize()
+                assert bf16_bits_equal(out, y_ref).all()
+    finally:
+        lib.mw8_set_tuning(-1, -1, -1)
+
+
+@pytest.mark.parametrize("act", ["silu", "gelu"])
+@pytest.mark.parametrize("routed", [False, True])
+def test_walk_activation_equals_separate(act, routed):
+    k, N, K, B = 2, 2048, 768, 64
+    ids, W, SW, tw, gen = _case(COUNTS, k, N, K, 11)
+    M, E = ids.shape[0], W.shape[0]
+    idsd, twd, Wd, SWd = ids.to(DEV), tw.to(DEV), W.to(DEV), (SW * 1e-2).to(DEV)
+    assert moe_gemm_act_preferred(M * k, N, K, E)
+    sorted_ids, expert_ids, npp = moe_align_block_size(idsd, B, E)
+    q, s = quant_per_token(torch.randn(M, K, generator=gen).to(torch.bfloat16).to(DEV))
+    announce(f"walk activation {act} routed={routed}")
+    lib = mw8lib.load()
+    try:
+        lib.mw8_set_tuning(-1, -1, 0)  # one tile per alignment block
+        c1 = torch.empty(M * k, N, dtype=torch.bfloat16, device=DEV)
+        fused_moe_kernel_w8a8(q, s, Wd, SWd, c1, twd, sorted_ids, expert_ids, npp, routed, k, B, M * k)
+        lib.mw8_set_tuning(-1, -1, 2)
+        out = torch.empty(M * k, N // 2, dtype=torch.bfloat16, device=DEV)
+        fused_moe_kernel_act_w8a8(q, s, Wd, SWd, out, sorted_ids, expert_ids, npp, k, B, M * k, act,
+                                  twd if routed else None)
+        torch.cuda.synchronize()
+    finally:
+        lib.mw8_set_tuning(-1, -1, -1)
+    want = act_and_mul_quant(c1, act, return_act=True)[2]
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+
+
+def test_walk_preference_is_host_only():
+    assert moe_gemm_act_preferred(2400, 1536, 2048, 128)
+    assert not moe_gemm_act_preferred(100, 1536, 512, 128)  # four K stages: below the walk's fewest
+    assert moe_gemm_act_preferred(32 * 128, 1536, 512, 128)
+    assert not moe_gemm_act_preferred(2400, 1536, 2040, 128)
