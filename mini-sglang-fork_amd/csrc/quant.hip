@@ -5,20 +5,23 @@
 // act_rows:     x bf16 [R, 2d] (gate | up) -> a = bf16(act(g) * u) ->
 //               quantized exactly as above; optionally also writes a.
 //
-// One row is owned by TPR threads (32 = half a wave, 64 = one wave, or 256 = four waves).
-// Each thread keeps VPT 16-byte vectors (8 bf16) of the row in registers,
-// so the row is read from HBM once: 16-byte coalesced loads, an integer
-// max over the sign-cleared bf16 bit patterns (monotone for finite
-// values), a wave/LDS max-reduction, then quantize-from-registers and
-// 8-byte stores.  Rows whose length exceeds TPR*VPT*8 take the generic
-// kernel, which re-reads the row (second read hits L2).
+// One row is owned by TPR threads: 16 or 32 (part of a wave, several rows
+// per wave), 64 (a wave, four rows per block), or 0 = the whole block, one
+// row per block of 128 - 1024 threads.  Each thread keeps VPT 16-byte
+// vectors (8 bf16) of the row in registers, so the row is read from HBM
+// once: 16-byte coalesced loads, an integer max over the sign-cleared bf16
+// bit patterns (monotone for finite values), a wave/LDS max-reduction, then
+// quantize-from-registers and 8-byte stores.  Rows past 32768 elements, or
+// off the vector alignment, take the generic kernel, which re-reads the row
+// (second read hits L2).
+#include <type_traits>
+
 #include "mw8_common.h"
 
 namespace mw8 {
 namespace {
 
 constexpr int kBlock = 256;
-
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
@@ -48,21 +51,39 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
   return v;
 }
 
-// Max over the TPR threads owning one row.  TPR == 32 / 64: lanes of a
-// half wave / the wave.  TPR == 256: one row per block, cross-wave through
-// LDS.
+// Threads per row and rows per block: TPR > 0 packs kBlock / TPR rows into a
+// block, TPR == 0 gives the block one row.
+template <int TPR>
+__device__ __forceinline__ int row_threads() { return TPR > 0 ? TPR : static_cast<int>(blockDim.x); }
+template <int TPR>
+__device__ __forceinline__ int64_t row_index() {
+  if constexpr (TPR > 0) return static_cast<int64_t>(blockIdx.x) * (kBlock / TPR) + threadIdx.x / TPR;
+  else return blockIdx.x;
+}
+template <int TPR>
+__device__ __forceinline__ int row_thread() {
+  if constexpr (TPR > 0) return threadIdx.x % TPR;
+  else return threadIdx.x;
+}
+constexpr int kMaxWaves = 16;  // waves of a whole-block row
+
+// Max over the threads owning one row: lanes of part of a wave or of the
+// wave, or (TPR == 0) the block, cross-wave through LDS.
 template <int TPR>
 __device__ __forceinline__ uint32_t row_max(uint32_t v, uint32_t* red) {
-  if constexpr (TPR <= 64) {
+  if constexpr (TPR > 0) {
     return wave_max_u32<TPR>(v);
   } else {
+    // all kMaxWaves entries are filled (wave 0 repeats its maximum past the
+    // block's waves) and read together: one LDS latency, no loop over waves
     v = wave_max_u32(v);
-    const int wave = threadIdx.x >> 6, base = (threadIdx.x / TPR) * (TPR / 64);  // the row's first wave
-    if ((threadIdx.x & 63) == 0) red[wave] = v;
+    const int t = threadIdx.x, waves = blockDim.x >> 6;
+    if ((t & 63) == 0) red[t >> 6] = v;
+    else if (t >= waves && t < kMaxWaves) red[t] = v;
     __syncthreads();
-    uint32_t m = red[base];
+    uint32_t m = red[0];
 #pragma unroll
-    for (int w = 1; w < TPR / 64; ++w) m = red[base + w] > m ? red[base + w] : m;
+    for (int w = 1; w < kMaxWaves; ++w) m = red[w] > m ? red[w] : m;
     return m;
   }
 }
@@ -77,18 +98,14 @@ __device__ __forceinline__ uint32_t absmax8(const U16x8& v, uint32_t m) {
   return m;
 }
 
-
-
-
 // ------------------------------------------------------------ quantizer
 template <int TPR, int VPT>
-__global__ __launch_bounds__(kBlock) void quant_rows_kernel(
+__global__ __launch_bounds__(TPR > 0 ? kBlock : 64 * kMaxWaves) void quant_rows_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, int64_t M, int64_t K,
     int8_t* __restrict__ q, int64_t ldq, float* __restrict__ s) {
-  __shared__ uint32_t red[kBlock / 64];
-  constexpr int kRowsPerBlock = kBlock / TPR;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * kRowsPerBlock + threadIdx.x / TPR;
-  const int t = threadIdx.x % TPR;
+  __shared__ __align__(16) uint32_t red[kMaxWaves];
+  const int64_t row = row_index<TPR>();
+  const int t = row_thread<TPR>(), tpr = row_threads<TPR>();
   const bool live = row < M;  // uniform per TPR lanes; every lane reaches row_max
   const int64_t nvec = K >> 3;
   const U16x8* xr = reinterpret_cast<const U16x8*>(x + (live ? row : 0) * ldx);
@@ -97,7 +114,7 @@ __global__ __launch_bounds__(kBlock) void quant_rows_kernel(
   uint32_t m = 0;
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
-    const int64_t idx = t + static_cast<int64_t>(i) * TPR;
+    const int64_t idx = t + static_cast<int64_t>(i) * tpr;
     if (live && idx < nvec) {
       v[i] = ld_row16(xr + idx);
       m = absmax8(v[i], m);
@@ -110,13 +127,13 @@ __global__ __launch_bounds__(kBlock) void quant_rows_kernel(
   if (rs.fast) {  // row-uniform: one branch per row, not a select per element
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-      const int64_t idx = t + static_cast<int64_t>(i) * TPR;
+      const int64_t idx = t + static_cast<int64_t>(i) * tpr;
       if (idx < nvec) st_row8(qr + idx, quant8<true>(v[i], rs));
     }
   } else {
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-      const int64_t idx = t + static_cast<int64_t>(i) * TPR;
+      const int64_t idx = t + static_cast<int64_t>(i) * tpr;
       if (idx < nvec) st_row8(qr + idx, quant8<false>(v[i], rs));
     }
   }
@@ -127,7 +144,7 @@ __global__ __launch_bounds__(kBlock) void quant_rows_kernel(
 __global__ __launch_bounds__(kBlock) void quant_rows_generic_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, int64_t M, int64_t K,
     int8_t* __restrict__ q, int64_t ldq, float* __restrict__ s) {
-  __shared__ uint32_t red[kBlock / 64];
+  __shared__ __align__(16) uint32_t red[kMaxWaves];
   const int64_t row = blockIdx.x;
   const uint16_t* xr = x + row * ldx;
   uint32_t m = 0;
@@ -135,7 +152,7 @@ __global__ __launch_bounds__(kBlock) void quant_rows_generic_kernel(
     uint32_t a = xr[k] & 0x7FFFu;
     m = a > m ? a : m;
   }
-  m = row_max<kBlock>(m, red);
+  m = row_max<0>(m, red);
   const RowScale rs = row_scale(bf16_to_f32(static_cast<uint16_t>(m)));
   for (int64_t k = threadIdx.x; k < K; k += kBlock)
     q[row * ldq + k] = static_cast<int8_t>(static_cast<int>(quant_div_rne(bf16_to_f32(xr[k]), rs)));
@@ -148,13 +165,12 @@ __global__ __launch_bounds__(kBlock) void quant_rows_generic_kernel(
 // to a tolerance, while the requant that follows is exact on its bf16 value.
 
 template <int TPR, int VPT, int ACT>
-__global__ __launch_bounds__(kBlock) void act_rows_kernel(
+__global__ __launch_bounds__(TPR > 0 ? kBlock : 64 * kMaxWaves) void act_rows_kernel(
     const uint16_t* __restrict__ x, int64_t R, int64_t d,
     int8_t* __restrict__ q, float* __restrict__ s, uint16_t* __restrict__ a_out) {
-  __shared__ uint32_t red[kBlock / 64];
-  constexpr int kRowsPerBlock = kBlock / TPR;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * kRowsPerBlock + threadIdx.x / TPR;
-  const int t = threadIdx.x % TPR;
+  __shared__ __align__(16) uint32_t red[kMaxWaves];
+  const int64_t row = row_index<TPR>();
+  const int t = row_thread<TPR>(), tpr = row_threads<TPR>();
   const bool live = row < R;
   const int64_t nvec = d >> 3;
   const U16x8* gr = reinterpret_cast<const U16x8*>(x + (live ? row : 0) * 2 * d);
@@ -164,7 +180,7 @@ __global__ __launch_bounds__(kBlock) void act_rows_kernel(
   uint32_t m = 0;
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
-    const int64_t idx = t + static_cast<int64_t>(i) * TPR;
+    const int64_t idx = t + static_cast<int64_t>(i) * tpr;
     if (live && idx < nvec) {
       const U16x8 g = ld_row16(gr + idx);
       const U16x8 u = ld_row16(ur + idx);
@@ -186,7 +202,7 @@ __global__ __launch_bounds__(kBlock) void act_rows_kernel(
   if (q == nullptr) {  // activation only (launch-uniform): no requant
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-      const int64_t idx = t + static_cast<int64_t>(i) * TPR;
+      const int64_t idx = t + static_cast<int64_t>(i) * tpr;
       if (idx < nvec) st_row16(ar + idx, v[i]);
     }
     return;
@@ -196,20 +212,20 @@ __global__ __launch_bounds__(kBlock) void act_rows_kernel(
   if (rs.fast) {
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-      const int64_t idx = t + static_cast<int64_t>(i) * TPR;
+      const int64_t idx = t + static_cast<int64_t>(i) * tpr;
       if (idx < nvec) st_row8(qr + idx, quant8<true>(v[i], rs));
     }
   } else {
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-      const int64_t idx = t + static_cast<int64_t>(i) * TPR;
+      const int64_t idx = t + static_cast<int64_t>(i) * tpr;
       if (idx < nvec) st_row8(qr + idx, quant8<false>(v[i], rs));
     }
   }
   if (ar) {
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-      const int64_t idx = t + static_cast<int64_t>(i) * TPR;
+      const int64_t idx = t + static_cast<int64_t>(i) * tpr;
       if (idx < nvec) st_row16(ar + idx, v[i]);
     }
   }
@@ -225,25 +241,27 @@ __global__ __launch_bounds__(kBlock) void act_rows_kernel(
 // only if y_out is given.  Replaces flashinfer rmsnorm / fused_add_rmsnorm
 // (python/minisgl/layers/norm.py:8-38) followed by the quantizer of the
 // next W8A8 linear.
+template <int W = 64>
 __device__ __forceinline__ double wave_sum_f64(double v) {
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
+  for (int off = W / 2; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
   return v;
 }
 
 template <int TPR>
 __device__ __forceinline__ double row_sum_f64(double v, double* red) {
-  v = wave_sum_f64(v);
-  if constexpr (TPR == 64) {
-    return v;
+  if constexpr (TPR > 0) {
+    return wave_sum_f64<TPR>(v);
   } else {
-    const int wave = threadIdx.x >> 6, base = (threadIdx.x / TPR) * (TPR / 64);  // the row's first wave
-    if ((threadIdx.x & 63) == 0) red[wave] = v;
+    v = wave_sum_f64(v);
+    const int t = threadIdx.x, waves = blockDim.x >> 6;
+    if ((t & 63) == 0) red[t >> 6] = v;
+    else if (t >= waves && t < kMaxWaves) red[t] = 0.0;
     __syncthreads();
-    double t = red[base];
+    double sum = red[0];
 #pragma unroll
-    for (int w = 1; w < TPR / 64; ++w) t += red[base + w];
-    return t;
+    for (int w = 1; w < kMaxWaves; ++w) sum += red[w];
+    return sum;
   }
 }
 
@@ -253,19 +271,20 @@ __device__ __forceinline__ double row_sum_f64(double v, double* red) {
 // matrix; a per-head view q.view(M, heads, D) of a row of qkv is inner =
 // heads, ld = qkv width.  residual, q and s are plain [M, H] / [M].
 template <int TPR, int VPT, bool RES, bool QUANT>
-__global__ __launch_bounds__(kBlock) void rmsnorm_rows_kernel(
+__global__ __launch_bounds__(TPR > 0 ? kBlock : 64 * kMaxWaves) void rmsnorm_rows_kernel(
     const uint16_t* x, uint16_t* __restrict__ res, const uint16_t* __restrict__ w,
     float eps, int64_t M, int64_t H, int8_t* __restrict__ q, float* __restrict__ s,
     uint16_t* y_out, int64_t inner, int64_t ldx, int64_t ldy) {
-  __shared__ double dred[kBlock / 64];
-  __shared__ uint32_t red[kBlock / 64];
-  constexpr int kRowsPerBlock = kBlock / TPR;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * kRowsPerBlock + threadIdx.x / TPR;
-  const int t = threadIdx.x % TPR;
-  const bool live = row < M;  // uniform per wave (TPR >= 64)
+  __shared__ double dred[kMaxWaves];
+  __shared__ __align__(16) uint32_t red[kMaxWaves];
+  const int64_t row = row_index<TPR>();
+  const int t = row_thread<TPR>(), tpr = row_threads<TPR>();
+  const bool live = row < M;  // uniform per row; every lane reaches the reductions
   const int64_t nvec = H >> 3;
   const int64_t lrow = live ? row : 0;
-  const int64_t grp = inner == 1 ? lrow : lrow / inner, sub = lrow - grp * inner;
+  // 32-bit division: the host keeps M below 2^31
+  const int64_t grp = inner == 1 ? lrow : static_cast<uint32_t>(lrow) / static_cast<uint32_t>(inner);
+  const int64_t sub = lrow - grp * inner;
   const U16x8* xr = reinterpret_cast<const U16x8*>(x + grp * ldx + sub * H);
   U16x8* rr = RES ? reinterpret_cast<U16x8*>(res + (live ? row : 0) * H) : nullptr;
   const U16x8* wr = reinterpret_cast<const U16x8*>(w);
@@ -274,7 +293,7 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_rows_kernel(
   double ss = 0.0;
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
-    const int64_t idx = t + static_cast<int64_t>(i) * TPR;
+    const int64_t idx = t + static_cast<int64_t>(i) * tpr;
     if (live && idx < nvec) {
       v[i] = ld_row16(xr + idx);
       if constexpr (RES) {
@@ -302,7 +321,7 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_rows_kernel(
   uint32_t m = 0;
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
-    const int64_t idx = t + static_cast<int64_t>(i) * TPR;
+    const int64_t idx = t + static_cast<int64_t>(i) * tpr;
     if (live && idx < nvec) {
       const U16x8 wv = wr[idx];
 #pragma unroll
@@ -322,13 +341,13 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_rows_kernel(
     if (rs.fast) {
 #pragma unroll
       for (int i = 0; i < VPT; ++i) {
-        const int64_t idx = t + static_cast<int64_t>(i) * TPR;
+        const int64_t idx = t + static_cast<int64_t>(i) * tpr;
         if (idx < nvec) st_row8(qr + idx, quant8<true>(v[i], rs));
       }
     } else {
 #pragma unroll
       for (int i = 0; i < VPT; ++i) {
-        const int64_t idx = t + static_cast<int64_t>(i) * TPR;
+        const int64_t idx = t + static_cast<int64_t>(i) * tpr;
         if (idx < nvec) st_row8(qr + idx, quant8<false>(v[i], rs));
       }
     }
@@ -338,91 +357,111 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_rows_kernel(
     U16x8* yr = reinterpret_cast<U16x8*>(y_out + grp * ldy + sub * H);
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-      const int64_t idx = t + static_cast<int64_t>(i) * TPR;
+      const int64_t idx = t + static_cast<int64_t>(i) * tpr;
       if (idx < nvec) st_row16(yr + idx, v[i]);
     }
   }
 }
 
-// Pick (TPR, VPT) for a row of nvec 16-byte vectors; false if none fits.
+// Pick (TPR, VPT) for rows of nvec 16-byte vectors; false if none fits.
+//
+// Measured on MI355X (graph nodes of 10 rotating inputs, us; the earlier
+// choice of 64 threads up to 512 vectors and 256 above -> this one).  Where
+// one thread per vector fits the chip's 512 Ki resident threads, every load
+// is in flight at once and the row's serial part (reductions, the quotient,
+// the activation) is shortest: quant 512 x 5120 5.1 -> 4.8, 777 x 3072 6.2
+// -> 4.8; gelu 777 x 3072 12.3 -> 7.6; silu 16 x 3072 7.2 -> 4.0, 2400 x
+// 768 5.8 -> 5.4; norm 300 x 2048 4.5 -> 3.8.  Longer rows take the fewest
+// vectors that 1024 threads hold (silu 64 x 17408 9.0 -> 7.1, quant 6.2 ->
+// 4.9 at one row), and 6 per thread past 512 rows (quant 2080 x 25600 39.7
+// -> 33.4, where blocks of 256 x 16 left 32 rows to a round of their own;
+// 8192 x 17408 75.7 -> 73.7).  Rows of 513 - 1024 vectors beyond the
+// resident threads: 6 per thread (quant 2080 x 6400 11.7 -> 10.1, norm 2080
+// x 5120 14.0 -> 12.7; one per thread 11.4 against 9.5 for 2080 x 5120), 3
+// or 4 from 4096 rows (norm + residual 8192 x 5120 53.6 against 56.5 with
+// 6, quant 6000 x 8192 28.2 with 4 against 29.4 with 3).
+// Up to 16 vectors four rows share a wave: the per-head norms (H = 128),
+// which kept 16 lanes of a wave busy, 2080 x 64 heads 46.2 -> 16.3 and 512 x
+// 40 heads 10.0 -> 4.8.
+constexpr int64_t kResidentThreads = 512 * 1024;
+
 template <template <int, int> class Launch, typename... Args>
 bool dispatch_rows(int64_t nvec, int64_t rows, hipStream_t st, Args... args) {
   auto go = [&](auto tpr_c, auto vpt_c) {
     constexpr int TPR = decltype(tpr_c)::value;
     constexpr int VPT = decltype(vpt_c)::value;
-    const int64_t blocks = (rows + (kBlock / TPR) - 1) / (kBlock / TPR);
-    Launch<TPR, VPT>::run(dim3(static_cast<unsigned>(blocks)), st, args...);
+    constexpr int kPerBlock = TPR > 0 ? kBlock / (TPR > 0 ? TPR : 1) : 1;
+    const int64_t threads = TPR > 0 ? kBlock : (nvec + 64 * VPT - 1) / (64 * VPT) * 64;
+    Launch<TPR, VPT>::run(dim3(static_cast<unsigned>((rows + kPerBlock - 1) / kPerBlock)),
+                          dim3(static_cast<unsigned>(threads)), st, args...);
     return true;
   };
+  using I0 = std::integral_constant<int, 0>;
+  using I16 = std::integral_constant<int, 16>;
   using I32 = std::integral_constant<int, 32>;
   using I64 = std::integral_constant<int, 64>;
-  using I256 = std::integral_constant<int, 256>;
-  // two rows per wave where that keeps more lanes busy than one (short
-  // rows: the MoE activation at I = 768 is 96 vectors, 75% of 64 x 2)
-  if constexpr (Launch<32, 1>::kHalfWaveRows) {
-    if (nvec <= 32) return go(I32{}, std::integral_constant<int, 1>{});
-    if (nvec > 64 && nvec <= 96) return go(I32{}, std::integral_constant<int, 3>{});
-  }
-  // few lanes idle on the last vector (K = 5120: 640 of 768 slots, K =
-  // 17408: 2176 of 2304).  Rows past 512 vectors use 256-thread rows: one
-  // wave per 5120-wide row measured slower for the fused RMSNorm.
-  if (nvec <= 64 * 1) return go(I64{}, std::integral_constant<int, 1>{});
-  if (nvec <= 64 * 2) return go(I64{}, std::integral_constant<int, 2>{});
-  if (nvec <= 64 * 3) return go(I64{}, std::integral_constant<int, 3>{});
-  if (nvec <= 64 * 4) return go(I64{}, std::integral_constant<int, 4>{});
-  if (nvec <= 64 * 6) return go(I64{}, std::integral_constant<int, 6>{});
-  if (nvec <= 64 * 8) return go(I64{}, std::integral_constant<int, 8>{});
-  if (nvec <= 256 * 3) return go(I256{}, std::integral_constant<int, 3>{});
-  if (nvec <= 256 * 4) return go(I256{}, std::integral_constant<int, 4>{});
-  if (nvec <= 256 * 6) return go(I256{}, std::integral_constant<int, 6>{});
-  if (nvec <= 256 * 8) return go(I256{}, std::integral_constant<int, 8>{});
-  if (nvec <= 256 * 9) return go(I256{}, std::integral_constant<int, 9>{});
-  if (nvec <= 256 * 12) return go(I256{}, std::integral_constant<int, 12>{});
-  if (nvec <= 256 * 16) return go(I256{}, std::integral_constant<int, 16>{});
-  return false;
+  using V1 = std::integral_constant<int, 1>;
+  using V2 = std::integral_constant<int, 2>;
+  using V3 = std::integral_constant<int, 3>;
+  using V4 = std::integral_constant<int, 4>;
+  using V6 = std::integral_constant<int, 6>;
+  using V8 = std::integral_constant<int, 8>;
+  if (nvec > 1024 * 4) return false;  // 32768 elements
+  if (nvec <= 16) return go(I16{}, V1{});
+  if (nvec <= 32) return go(I32{}, V1{});
+  if (nvec <= 64) return go(I64{}, V1{});
+  if (nvec > 1024) return rows <= 512 ? go(I0{}, V4{}) : go(I0{}, V6{});
+  if (rows * nvec <= kResidentThreads) return go(I0{}, V1{});
+  // two rows per wave where that keeps more lanes busy than one (the MoE
+  // activation at I = 768 is 96 vectors, 75% of 64 x 2)
+  if (nvec <= 96) return go(I32{}, V3{});
+  if (nvec <= 64 * 2) return go(I64{}, V2{});
+  if (nvec <= 64 * 3) return go(I64{}, V3{});
+  if (nvec <= 64 * 4) return go(I64{}, V4{});
+  if (nvec <= 64 * 6) return go(I64{}, V6{});
+  if (nvec <= 64 * 8) return go(I64{}, V8{});
+  if (rows < 4096) return go(I0{}, V6{});
+  return nvec <= 768 ? go(I0{}, V3{}) : go(I0{}, V4{});  // up to 256 threads
 }
 
 template <int TPR, int VPT>
 struct QuantLaunch {
-  static constexpr bool kHalfWaveRows = true;
-  static void run(dim3 grid, hipStream_t st, const uint16_t* x, int64_t ldx, int64_t M,
+  static void run(dim3 grid, dim3 block, hipStream_t st, const uint16_t* x, int64_t ldx, int64_t M,
                   int64_t K, int8_t* q, int64_t ldq, float* s) {
-    hipLaunchKernelGGL((quant_rows_kernel<TPR, VPT>), grid, dim3(kBlock), 0, st, x, ldx, M, K,
+    hipLaunchKernelGGL((quant_rows_kernel<TPR, VPT>), grid, block, 0, st, x, ldx, M, K,
                        q, ldq, s);
   }
 };
 
 template <int TPR, int VPT>
 struct ActLaunch {
-  static constexpr bool kHalfWaveRows = true;
-  static void run(dim3 grid, hipStream_t st, const uint16_t* x, int64_t R, int64_t d, int act,
+  static void run(dim3 grid, dim3 block, hipStream_t st, const uint16_t* x, int64_t R, int64_t d, int act,
                   int8_t* q, float* s, uint16_t* a_out) {
     if (act == 0)
-      hipLaunchKernelGGL((act_rows_kernel<TPR, VPT, 0>), grid, dim3(kBlock), 0, st, x, R, d, q, s,
+      hipLaunchKernelGGL((act_rows_kernel<TPR, VPT, 0>), grid, block, 0, st, x, R, d, q, s,
                          a_out);
     else
-      hipLaunchKernelGGL((act_rows_kernel<TPR, VPT, 1>), grid, dim3(kBlock), 0, st, x, R, d, q, s,
+      hipLaunchKernelGGL((act_rows_kernel<TPR, VPT, 1>), grid, block, 0, st, x, R, d, q, s,
                          a_out);
   }
 };
 
 template <int TPR, int VPT>
 struct NormLaunch {
-  static constexpr bool kHalfWaveRows = false;
-  static void run(dim3 grid, hipStream_t st, const uint16_t* x, uint16_t* res, const uint16_t* w,
+  static void run(dim3 grid, dim3 block, hipStream_t st, const uint16_t* x, uint16_t* res, const uint16_t* w,
                   float eps, int64_t M, int64_t H, int8_t* q, float* s, uint16_t* y, int64_t inner,
                   int64_t ldx, int64_t ldy) {
     if (res && q)
-      hipLaunchKernelGGL((rmsnorm_rows_kernel<TPR, VPT, true, true>), grid, dim3(kBlock), 0, st, x, res,
+      hipLaunchKernelGGL((rmsnorm_rows_kernel<TPR, VPT, true, true>), grid, block, 0, st, x, res,
                          w, eps, M, H, q, s, y, inner, ldx, ldy);
     else if (res)
-      hipLaunchKernelGGL((rmsnorm_rows_kernel<TPR, VPT, true, false>), grid, dim3(kBlock), 0, st, x, res,
+      hipLaunchKernelGGL((rmsnorm_rows_kernel<TPR, VPT, true, false>), grid, block, 0, st, x, res,
                          w, eps, M, H, q, s, y, inner, ldx, ldy);
     else if (q)
-      hipLaunchKernelGGL((rmsnorm_rows_kernel<TPR, VPT, false, true>), grid, dim3(kBlock), 0, st, x, res,
+      hipLaunchKernelGGL((rmsnorm_rows_kernel<TPR, VPT, false, true>), grid, block, 0, st, x, res,
                          w, eps, M, H, q, s, y, inner, ldx, ldy);
     else
-      hipLaunchKernelGGL((rmsnorm_rows_kernel<TPR, VPT, false, false>), grid, dim3(kBlock), 0, st, x, res,
+      hipLaunchKernelGGL((rmsnorm_rows_kernel<TPR, VPT, false, false>), grid, block, 0, st, x, res,
                          w, eps, M, H, q, s, y, inner, ldx, ldy);
   }
 };
