@@ -17,8 +17,36 @@ from .lib import check, load
 _ACT = {"silu": 0, "gelu": 1}
 
 
+# The current stream's handle and the current device as integers, without
+# the Stream and device objects of torch.cuda.current_stream (1.9 us a call)
+# and torch.cuda.device (1.4 us): an eager decode call is a few launches of
+# 5-10 us each, and its host time is what bounds it.
+_raw_stream = torch._C._cuda_getCurrentRawStream
+_get_device = torch._C._cuda_getDevice
+
+
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.get_device())
+
+
+class _Stay:
+    """The device guard of a call whose tensors are on the current device."""
+
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_STAY = _Stay()
+
+
+def _device_of(t: torch.Tensor):
+    """A context in which t's device is current (the library plans for the
+    current device)."""
+    index = t.get_device()
+    return _STAY if _get_device() == index else torch.cuda.device(index)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -37,8 +65,16 @@ def _on_gpu(*ts: Optional[torch.Tensor]) -> None:
 
 
 def _same_device(*ts: Optional[torch.Tensor]) -> None:
-    devs = {t.device for t in ts if t is not None}
-    if len(devs) > 1:
+    dev = None
+    same = True
+    for t in ts:
+        if t is not None:
+            if dev is None:
+                dev = t.device
+            elif t.device != dev:
+                same = False
+    if not same:
+        devs = {t.device for t in ts if t is not None}
         raise ValueError(f"the W8A8 HIP path needs every tensor on one device, got {sorted(map(str, devs))}")
 
 
@@ -71,16 +107,15 @@ def reserve_gemm_workspace(device: torch.device) -> torch.Tensor:
     return ws
 
 
-def _call_workspace(M: int, N: int, K: int, device: torch.device) -> Optional[torch.Tensor]:
-    """The K split's int32 partial tiles for one call at (M, N, K), or None
-    when no split applies: a buffer from torch's caching allocator, which
-    hands a freed block back only to work ordered after its last use on the
-    same stream (and takes it from the graph's private pool under capture),
-    so calls on concurrent streams never share one.  The size is planned for
-    q's device and the calling thread's tuning override, as the call is."""
-    with torch.cuda.device(device):
-        need = int(load().mw8_gemm_workspace_bytes(M, N, K))
-    return torch.empty(need, dtype=torch.uint8, device=device) if need > 0 else None
+def _call_workspace(need: int, like: torch.Tensor) -> Optional[torch.Tensor]:
+    """The K split's int32 partial tiles for one call (None if it needs
+    none): a buffer from torch's caching allocator, which hands a freed block
+    back only to work ordered after its last use on the same stream (and
+    takes it from the graph's private pool under capture), so calls on
+    concurrent streams never share one.  The caller asks for the size within
+    the device context of the call and under the calling thread's tuning
+    override, as the call itself plans it."""
+    return torch.empty(need, dtype=torch.uint8, device=like.device) if need > 0 else None
 
 
 def gemm_workspace(M: int, N: int, K: int, device: torch.device) -> Optional[torch.Tensor]:
@@ -100,10 +135,16 @@ def quant_per_token(
     _need(x.dtype == torch.bfloat16 and x.dim() == 2, "quant_per_token: x must be bf16 [M, K]")
     _need(x.stride(1) == 1, "quant_per_token: last dim must be contiguous")
     M, K = x.shape
-    q = out if out is not None else torch.empty((M, K), dtype=torch.int8, device=x.device)
-    s = scale if scale is not None else torch.empty((M,), dtype=torch.float32, device=x.device)
-    _need(q.dtype == torch.int8 and q.shape == (M, K) and q.stride(1) == 1, "bad q buffer")
-    _need(s.dtype == torch.float32 and s.shape == (M,) and s.is_contiguous(), "bad s buffer")
+    if out is None:
+        q = torch.empty((M, K), dtype=torch.int8, device=x.device)
+    else:
+        q = out
+        _need(q.dtype == torch.int8 and q.shape == (M, K) and q.stride(1) == 1, "bad q buffer")
+    if scale is None:
+        s = torch.empty((M,), dtype=torch.float32, device=x.device)
+    else:
+        s = scale
+        _need(s.dtype == torch.float32 and s.shape == (M,) and s.is_contiguous(), "bad s buffer")
     if M == 0:
         return q, s
     check(
@@ -254,13 +295,15 @@ def gemm_w8a8(
     if bias is not None:
         _need(bias.dtype == torch.bfloat16 and bias.shape == (N,) and bias.is_contiguous(), "bias: bf16 [N]")
     y = out if out is not None else torch.empty((M, N), dtype=torch.bfloat16, device=q.device)
-    _need(y.dtype == torch.bfloat16 and y.shape == (M, N) and y.is_contiguous(), "bad out buffer")
+    if out is not None:
+        _need(y.dtype == torch.bfloat16 and y.shape == (M, N) and y.is_contiguous(), "bad out buffer")
     if M == 0:
         return y
-    ws = _call_workspace(M, N, K, q.device)
-    with torch.cuda.device(q.device):  # the library plans the tiling for the current device
+    lib = load()
+    with _device_of(q):  # the library plans the tiling for the current device
+        ws = _call_workspace(lib.mw8_gemm_workspace_bytes(M, N, K), q)
         check(
-            load().mw8_gemm_w8a8_bf16(
+            lib.mw8_gemm_w8a8_bf16(
                 _ptr(q), _ptr(s_a), _ptr(w), _ptr(s_w), _ptr(bias), _ptr(y), M, N, K, _ptr(ws),
                 0 if ws is None else ws.numel(), _stream(q),
             )
@@ -307,12 +350,11 @@ def gemm_act_w8a8(
     _need(y.dtype == torch.bfloat16 and y.shape == (M, I) and y.is_contiguous(), "bad out buffer")
     if M == 0:
         return y
-    with torch.cuda.device(q.device):
-        need = int(load().mw8_gemm_act_workspace_bytes(M, I, K))
-    ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need > 0 else None
-    with torch.cuda.device(q.device):
+    lib = load()
+    with _device_of(q):
+        ws = _call_workspace(lib.mw8_gemm_act_workspace_bytes(M, I, K), q)
         check(
-            load().mw8_gemm_act_w8a8_bf16(
+            lib.mw8_gemm_act_w8a8_bf16(
                 _ptr(q), _ptr(s_a), _ptr(w), _ptr(s_w), _ACT[activation], _ptr(y), M, I, K, _ptr(ws),
                 0 if ws is None else ws.numel(), _stream(q),
             )
@@ -362,10 +404,11 @@ def gemm_w8a8_i32(q: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     acc = torch.empty((M, N), dtype=torch.int32, device=q.device)
     if M == 0:
         return acc
-    ws = _call_workspace(M, N, K, q.device)
-    with torch.cuda.device(q.device):
+    lib = load()
+    with _device_of(q):
+        ws = _call_workspace(lib.mw8_gemm_workspace_bytes(M, N, K), q)
         check(
-            load().mw8_gemm_w8a8_i32(
+            lib.mw8_gemm_w8a8_i32(
                 _ptr(q), _ptr(w), _ptr(acc), M, N, K, _ptr(ws), 0 if ws is None else ws.numel(),
                 _stream(q),
             )

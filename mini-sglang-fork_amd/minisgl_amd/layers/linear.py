@@ -82,8 +82,7 @@ class _LinearW8A8Impl(BaseOP):
         return self._wpad
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        lead = x.shape[:-1]
-        x2 = x.reshape(-1, x.shape[-1])
+        x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
         M, K = x2.shape
         N = self.weight.shape[0]
         if (
@@ -104,7 +103,7 @@ class _LinearW8A8Impl(BaseOP):
         else:
             q, s = quant_per_token(x2)
             y = self.forward_quantized(q, s)
-        return y.view(*lead, y.shape[-1])
+        return y if x.dim() == 2 else y.view(*x.shape[:-1], N)
 
     def load_float_weight(self, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> None:
         """Quantize a bf16 [N, K] weight on the device into this layer."""
