@@ -346,6 +346,23 @@ constexpr KsplitCfg kKsplitCfgs[] = {
 constexpr int kNumKsplitCfgs = sizeof(kKsplitCfgs) / sizeof(kKsplitCfgs[0]);
 constexpr int kNumTileCfgs = kNumRingCfgs + kNumKsplitCfgs;
 
+// The 192 x 256 ring (8 waves 2x4 of 96 x 64, 2 A and 3 W slots with the
+// weight lead): three quarters of a 256 x 256 tile in three quarters of its
+// time, for row counts that 256-row tiles cover badly.  At 2080 rows those
+// leave their ninth row tile 32 rows deep, and N = 5120 gets 180 tiles for
+// 256 CUs where 192-row tiles give 220.  MI355X, weights from HBM, the earlier
+// choice -> 192 x 256, us: 2080 x 5120 x 25600 270 -> 233, x 17408 185 -> 160,
+// x 8192 92 -> 80, x 5120 62 -> 54; 2080 x 10240 x 5120 119 -> 108; 2080 x
+// 51200 x 5120 505 -> 498; 1500 x 7168 x 5120 65 -> 55; 3000 x 7168 x 5120 130
+// -> 105; 1024 x 10240 x 5120 68 -> 58; 300 x 34816 x 5120 93 -> 84.  Where
+// 256-row tiles fill whole waves it loses (4096 x 34816 x 5120 600 -> 646).
+// Its index follows the split-K tilings.
+constexpr TileCfg kRing192 = {192, 256, true, 128, 1, true, "tile3_gemm_kernel<192, 256, 128, 2, 4, 2>"};
+constexpr int kCfg192 = kNumTileCfgs;
+
+constexpr bool is_ksplit(int cfg) { return cfg >= kNumRingCfgs && cfg < kNumTileCfgs; }
+constexpr const TileCfg& ring_cfg(int cfg) { return cfg == kCfg192 ? kRing192 : kTileCfgs[cfg]; }
+
 constexpr int ksplit_sk(const KsplitCfg& c) { return c.kg * c.ks * 32; }
 
 // Column ranges of a ksplit grid over N: the fewest whose boundaries are
@@ -428,10 +445,17 @@ constexpr ModelCfg kModelCfgs[] = {
     {5, 3.0, 3.36, 3.36},   // 64x128, 4 stages
     {3, 6.0, 8.0, 8.0},     // 256x128, 8 waves, 3 stages (no K split): grids of 129-256 tiles
     {6, 5.0, 9.2, 9.2},     // 256x320, 8 waves 2x4 (near-ties go to 256x256)
+    // 192x256, 8 waves 2x4, weight lead: at this rate the 23 shapes measured
+    // 2-18% faster on it are picked (1-3% above it, 2600 x 5120 x 17408 and 7000
+    // x 7168 x 5120 are too, 4% and 1% slower; below, 300 x 34816 x 5120 is lost)
+    {kCfg192, 5.0, 9.3, 9.3},
 };
+constexpr const ModelCfg& kModel256 = kModelCfgs[0];
+constexpr const ModelCfg& kModel192 = kModelCfgs[6];
+static_assert(kModel256.cfg == 2 && kModel192.cfg == kCfg192, "model order");
 
 double model_us(int64_t M, int64_t N, int64_t K, const ModelCfg& mc) {
-  const TileCfg& t = kTileCfgs[mc.cfg];
+  const TileCfg& t = ring_cfg(mc.cfg);
   const int64_t cus = device_cus();
   const int64_t T = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
   const int64_t slots = cus * t.per_cu;
@@ -506,7 +530,14 @@ int default_tile_cfg(int64_t M, int64_t N, int64_t K) {
   int best = 1;
   double best_us = 1e300;
   for (const ModelCfg& mc : kModelCfgs) {
-    if (K % kTileCfgs[mc.cfg].bk != 0) continue;
+    if (K % ring_cfg(mc.cfg).bk != 0) continue;
+    if (mc.cfg == kCfg192) {
+      // not where every tile would split along K: the other tilings' splits
+      // are as fast or faster (800 x 5120 x 17408 109 against 103 us, 1024 x
+      // 5120 x 25600 159 against 144, 512 x 5120 x 17408 level)
+      const SplitPlan sp = plan_split(M, N, K, kRing192);
+      if (sp.sp > 1 && sp.full == 0) continue;
+    }
     const double us = model_us(M, N, K, mc);
     if (us < best_us) {
       best_us = us;
@@ -522,8 +553,8 @@ int default_tile_cfg(int64_t M, int64_t N, int64_t K) {
 
 // The ring configuration a dense call at (M, N, K) runs (override first).
 bool tile_cfg_fits(int cfg, int64_t M, int64_t N, int64_t K) {
-  if (cfg < 0 || cfg >= kNumTileCfgs) return false;
-  if (cfg < kNumRingCfgs) return !kTileCfgs[cfg].dma || K % kTileCfgs[cfg].bk == 0;
+  if (cfg < 0 || cfg > kCfg192) return false;
+  if (!is_ksplit(cfg)) return !ring_cfg(cfg).dma || K % ring_cfg(cfg).bk == 0;
   const KsplitCfg& c = kKsplitCfgs[cfg - kNumRingCfgs];
   int64_t gm = 0;
   return K % ksplit_sk(c) == 0 && ksplit_ranges(M, N, c, gm) > 0;
@@ -609,8 +640,8 @@ bool stream_fits(const GemmArgs& g) {
 template <int EPI>
 int dispatch_tile(GemmArgs g, void* ws, size_t ws_bytes, hipStream_t st) {
   const int cfg = select_tile_cfg(g.M, g.N, g.K);
-  if (cfg >= kNumRingCfgs) return dispatch_ksplit<EPI>(cfg - kNumRingCfgs, g, st);
-  const TileCfg c = kTileCfgs[cfg];
+  if (is_ksplit(cfg)) return dispatch_ksplit<EPI>(cfg - kNumRingCfgs, g, st);
+  const TileCfg c = ring_cfg(cfg);
   const int64_t tiles64 = ((g.M + c.bm - 1) / c.bm) * ((g.N + c.bn - 1) / c.bn);
   // the tile walk computes in 32 bits; a K split multiplies the blocks by at most 16
   MW8_REQUIRE(tiles64 <= (int64_t{1} << 26), kErrShape, "gemm: %lld output tiles exceed the tile walk's range",
@@ -649,6 +680,7 @@ int dispatch_tile(GemmArgs g, void* ws, size_t ws_bytes, hipStream_t st) {
                    : launch_tile3<64, 128, 128, 1, 4, 4, EPI, DenseRows, 0, kLeadSmall>(g, dim3(tiles), st);
       break;
     case 6: rc = launch_tile3<256, 320, 128, 2, 4, 2, EPI, DenseRows>(g, dim3(tiles), st); break;
+    case kCfg192: rc = launch_tile3<192, 256, 128, 2, 4, 2, EPI, DenseRows, 0, kLead256>(g, dim3(tiles), st); break;
     default: {
       const int64_t cus = device_cus();
       if (EPI == kEpiBf16 && tiles >= cus && stream_fits(g))
@@ -662,6 +694,7 @@ int dispatch_tile(GemmArgs g, void* ws, size_t ws_bytes, hipStream_t st) {
   switch (c.bm * 1000 + c.bn) {
     case 64128: return launch_split_reduce<64, 128, EPI>(g, sp, st);
     case 128128: return launch_split_reduce<128, 128, EPI>(g, sp, st);
+    case 192256: return launch_split_reduce<192, 256, EPI>(g, sp, st);
     default: return launch_split_reduce<256, 256, EPI>(g, sp, st);
   }
 }
@@ -792,7 +825,7 @@ int tuning_count(int kind);
 size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0 || !use_tile_path(M, N, K)) return 0;
   const int cfg = select_tile_cfg(M, N, K);
-  return cfg < kNumRingCfgs ? plan_split(M, N, K, kTileCfgs[cfg]).ws : 0;
+  return is_ksplit(cfg) ? 0 : plan_split(M, N, K, ring_cfg(cfg)).ws;
 }
 
 size_t gemm_workspace_max_bytes() {
@@ -827,7 +860,9 @@ int gemm_w8a8_i32(const int8_t* A, const int8_t* W, int32_t* acc, int64_t M, int
 namespace {
 int act_tile_cfg(int64_t M, int64_t N2, int64_t K) {
   const int cfg = select_tile_cfg(M, N2, K);
-  if (cfg == 2 || cfg == 3 || cfg == 4 || cfg == 5) return cfg;
+  // near ties (3%) stay on the 256x256 tiles, whose operand stream is smaller
+  if (cfg == kCfg192 && g_tile_cfg < 0 && 1.03 * model_us(M, N2, K, kModel192) > model_us(M, N2, K, kModel256)) return 2;
+  if (cfg == 2 || cfg == 3 || cfg == 4 || cfg == 5 || cfg == kCfg192) return cfg;
   if (cfg == 6 || cfg == 7) return 2;  // the 256x320 ring and the stream walk: 256x256
   return M > 128 ? 2 : 4;
 }
@@ -856,12 +891,14 @@ int dispatch_act(const GemmArgs& g, int cfg, unsigned tiles, bool split, const S
     case 3: rc = launch_tile3_act<256, 128, 4, 2, 3, kAct>(g, tiles, st); break;
     case 4: rc = launch_tile3_act<128, 128, 2, 2, 2, kAct, kLeadSmall>(g, tiles, st); break;
     case 5: rc = launch_tile3_act<64, 128, 1, 4, 4, kAct, kLeadSmall>(g, tiles, st); break;
+    case kCfg192: rc = launch_tile3_act<192, 256, 2, 4, 2, kAct, kLead256>(g, tiles, st); break;
     default: rc = launch_tile3_act<256, 256, 2, 4, 2, kAct, kLead256>(g, tiles, st); break;
   }
   if (rc != kOk || !split) return rc;
   switch (cfg) {
     case 4: return launch_split_reduce_act<128, 128, kAct>(g, sp, st);
     case 5: return launch_split_reduce_act<64, 128, kAct>(g, sp, st);
+    case kCfg192: return launch_split_reduce_act<192, 256, kAct>(g, sp, st);
     default: return launch_split_reduce_act<256, 256, kAct>(g, sp, st);
   }
 }
@@ -878,7 +915,7 @@ int gemm_act_cfg(int64_t M, int64_t I, int64_t K) {
 
 size_t gemm_act_workspace_bytes(int64_t M, int64_t I, int64_t K) {
   const int cfg = gemm_act_cfg(M, I, K);
-  return cfg < 0 ? 0 : plan_split(M, 2 * I, K, kTileCfgs[cfg]).ws;
+  return cfg < 0 ? 0 : plan_split(M, 2 * I, K, ring_cfg(cfg)).ws;
 }
 
 int gemm_act_w8a8_bf16(const int8_t* A, const float* sa, const int8_t* W, const float* sw, int act, void* y,
@@ -900,7 +937,7 @@ int gemm_act_w8a8_bf16(const int8_t* A, const float* sa, const int8_t* W, const 
   g.out = y; g.M = M; g.N = 2 * I; g.K = K; g.lda = K; g.ldo = I;
   g.top_k = 1;
   g.staged_out = 1;
-  const TileCfg c = kTileCfgs[cfg];
+  const TileCfg c = ring_cfg(cfg);
   const int64_t tiles64 = ((M + c.bm - 1) / c.bm) * ((2 * I + c.bn - 1) / c.bn);
   MW8_REQUIRE(tiles64 <= (int64_t{1} << 26), kErrShape, "gemm_act: %lld output tiles exceed the tile walk's range",
               (long long)tiles64);
@@ -1055,8 +1092,8 @@ const char* gemm_kernel_name(int64_t M, int64_t N, int64_t K) {
     return kDecodeCfgs[cfg].core == 0 ? "decode_gemm_kernel" : "decode3_gemm_kernel";
   }
   const int cfg = select_tile_cfg(M, N, K);
-  if (cfg >= kNumRingCfgs) return kKsplitCfgs[cfg - kNumRingCfgs].name;
-  return kTileCfgs[cfg].name;
+  if (is_ksplit(cfg)) return kKsplitCfgs[cfg - kNumRingCfgs].name;
+  return ring_cfg(cfg).name;
 }
 
 int tuning_count(int kind) {
