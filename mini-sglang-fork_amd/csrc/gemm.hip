@@ -295,15 +295,30 @@ int launch_tile3(const GemmArgs& g, dim3 grid, hipStream_t st) {
   return kOk;
 }
 
+// The 256 x 128 ring splits grids of up to 64 tiles, into four K ranges and
+// more.  At 129 - 256 rows it writes half the partial tiles of 256 x 256 (N =
+// 5120: 31 MB against 63) and reads half the token rows of 128 x 128.
+// MI355X, weights from HBM, us, the earlier choice -> 256 x 128 split: 256 x
+// 5120 x 17408 49.0 -> 42.4, 200 rows 46.2 -> 40.2; 400 x 3000 x 16384 48.0 ->
+// 39.7; 512 x 4096 x 12288 46.7 -> 42.1; 700 x 2048 x 16384 47.1 -> 43.5.  With
+// three ranges it is level or slower (512 x 5120 x 17408 69.4 -> 67.6, x 25600
+// 87.4 -> 95.4), with two slower (768 x 5120 x 17408 82.9 -> 86.7): the operand
+// stream, half as much again per output as in 256 x 256, then outweighs the
+// partial tiles.  One row tile does not stream its weights here: 256 x 5120 x
+// 17408 42.4 -> 41.6 from HBM, but 41.2 -> 45.4 with the weights in the MALL.
+constexpr int kMinRanges256x128 = 4;
+
 // 0: register-staged tile core (any K % 16 == 0); 1 and up: direct-to-LDS
 // ring (K % bk == 0).  per_cu: resident blocks per CU (LDS-bound); split:
-// the K split of the last partial wave applies.
+// the K split of the last partial wave applies; min_ranges: fewest K ranges
+// of such a split (from 3 up, only grids smaller than the chip split).
 struct TileCfg {
   int bm, bn;
   bool dma;
   int bk, per_cu;
   bool split;
-  const char* name;  // kernel name with its leading template arguments, as a trace shows it
+  const char* name;    // kernel name with its leading template arguments, as a trace shows it
+  int min_ranges = 2;
 };
 constexpr TileCfg kTileCfgs[] = {
     // 0: register-staged, 4 waves
@@ -313,8 +328,9 @@ constexpr TileCfg kTileCfgs[] = {
     // 2: ring, 8 waves (2x4 of 128 x 64), 2 stages (the weight stages a
     // stage further ahead, in a ring of 3: kLead256)
     {256, 256, true, 128, 1, true, "tile3_gemm_kernel<256, 256, 128, 2, 4, 2>"},
-    // 3: ring, 8 waves (4x2), 3 stages: grids of 129-256 tiles
-    {256, 128, true, 128, 1, false, "tile3_gemm_kernel<256, 128, 128, 4, 2, 3>"},
+    // 3: ring, 8 waves (4x2), 3 stages: grids of 129-256 tiles, and up to 64
+    // tiles split along K (kMinRanges256x128)
+    {256, 128, true, 128, 1, true, "tile3_gemm_kernel<256, 128, 128, 4, 2, 3>", kMinRanges256x128},
     // 4: ring, 4 waves (2x2), 2 stages (weight lead: kLeadSmall), two per CU
     {128, 128, true, 128, 2, true, "tile3_gemm_kernel<128, 128, 128, 2, 2, 2>"},
     // 5: ring, 4 waves (1x4), 4 stages (weight lead: kLeadSmall)
@@ -410,7 +426,7 @@ SplitPlan plan_split(int64_t M, int64_t N, int64_t K, const TileCfg& c) {
   const int64_t nkt = K / c.bk;
   if (sp > nkt) sp = nkt;
   if (sp > 16) sp = 16;
-  if (sp < 2 || (T >= slots && sp < 3)) return p;
+  if (sp < c.min_ranges || (T >= slots && (sp < 3 || c.min_ranges > 2))) return p;
   p.full = T - r;
   p.tail = r;
   p.sp = static_cast<int>(sp);
@@ -443,7 +459,7 @@ constexpr ModelCfg kModelCfgs[] = {
     {4, 3.0, 3.7, 6.1},     // 128x128 BK 128, 2 stages, two per CU
     {1, 3.0, 4.6, 5.9},     // 128x128 BK 64, 4 stages, two per CU
     {5, 3.0, 3.36, 3.36},   // 64x128, 4 stages
-    {3, 6.0, 8.0, 8.0},     // 256x128, 8 waves, 3 stages (no K split): grids of 129-256 tiles
+    {3, 6.0, 8.0, 8.0},     // 256x128, 8 waves, 3 stages: grids of 129-256 tiles, K splits of up to 64
     {6, 5.0, 9.2, 9.2},     // 256x320, 8 waves 2x4 (near-ties go to 256x256)
     // 192x256, 8 waves 2x4, weight lead: at this rate the 23 shapes measured
     // 2-18% faster on it are picked (1-3% above it, 2600 x 5120 x 17408 and 7000
@@ -695,6 +711,7 @@ int dispatch_tile(GemmArgs g, void* ws, size_t ws_bytes, hipStream_t st) {
     case 64128: return launch_split_reduce<64, 128, EPI>(g, sp, st);
     case 128128: return launch_split_reduce<128, 128, EPI>(g, sp, st);
     case 192256: return launch_split_reduce<192, 256, EPI>(g, sp, st);
+    case 256128: return launch_split_reduce<256, 128, EPI>(g, sp, st);
     default: return launch_split_reduce<256, 256, EPI>(g, sp, st);
   }
 }
@@ -897,6 +914,7 @@ int dispatch_act(const GemmArgs& g, int cfg, unsigned tiles, bool split, const S
   if (rc != kOk || !split) return rc;
   switch (cfg) {
     case 4: return launch_split_reduce_act<128, 128, kAct>(g, sp, st);
+    case 3: return launch_split_reduce_act<256, 128, kAct>(g, sp, st);
     case 5: return launch_split_reduce_act<64, 128, kAct>(g, sp, st);
     case kCfg192: return launch_split_reduce_act<192, 256, kAct>(g, sp, st);
     default: return launch_split_reduce_act<256, 256, kAct>(g, sp, st);
