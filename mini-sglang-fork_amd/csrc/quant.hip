@@ -373,9 +373,11 @@ __global__ __launch_bounds__(TPR > 0 ? kBlock : 64 * kMaxWaves) void rmsnorm_row
 // -> 4.8; gelu 777 x 3072 12.3 -> 7.6; silu 16 x 3072 7.2 -> 4.0, 2400 x
 // 768 5.8 -> 5.4; norm 300 x 2048 4.5 -> 3.8.  Longer rows take the fewest
 // vectors that 1024 threads hold (silu 64 x 17408 9.0 -> 7.1, quant 6.2 ->
-// 4.9 at one row), and 6 per thread past 512 rows (quant 2080 x 25600 39.7
-// -> 33.4, where blocks of 256 x 16 left 32 rows to a round of their own;
-// 8192 x 17408 75.7 -> 73.7).  Rows of 513 - 1024 vectors beyond the
+// 4.9 at one row), and past 512 rows 3, 5, 7 or 8 in blocks of up to 512
+// threads: quant 2080 x 25600 39.2 -> 33.2 (7; blocks of 256 x 16 left 32
+// rows to a round of their own), 5000 x 25600 76.7 -> 68.6, 8192 x 17408 77.2
+// -> 75.4 (5; 3, 4, 6, 7 80.4, 77.4, 77.0, 79.0), 8192 x 12288 53.0 -> 50.6
+// (3; 5 53.6).  Rows of 513 - 1024 vectors beyond the
 // resident threads: 6 per thread (quant 2080 x 6400 11.7 -> 10.1, norm 2080
 // x 5120 14.0 -> 12.7; one per thread 11.4 against 9.5 for 2080 x 5120), 3
 // or 4 from 4096 rows (norm + residual 8192 x 5120 53.6 against 56.5 with
@@ -404,13 +406,20 @@ bool dispatch_rows(int64_t nvec, int64_t rows, hipStream_t st, Args... args) {
   using V2 = std::integral_constant<int, 2>;
   using V3 = std::integral_constant<int, 3>;
   using V4 = std::integral_constant<int, 4>;
+  using V5 = std::integral_constant<int, 5>;
   using V6 = std::integral_constant<int, 6>;
+  using V7 = std::integral_constant<int, 7>;
   using V8 = std::integral_constant<int, 8>;
   if (nvec > 1024 * 4) return false;  // 32768 elements
   if (nvec <= 16) return go(I16{}, V1{});
   if (nvec <= 32) return go(I32{}, V1{});
   if (nvec <= 64) return go(I64{}, V1{});
-  if (nvec > 1024) return rows <= 512 ? go(I0{}, V4{}) : go(I0{}, V6{});
+  if (nvec > 1024) {
+    if (rows <= 512) return go(I0{}, V4{});
+    if (nvec <= 512 * 3) return go(I0{}, V3{});
+    if (nvec <= 512 * 5) return go(I0{}, V5{});
+    return nvec <= 512 * 7 ? go(I0{}, V7{}) : go(I0{}, V8{});
+  }
   if (rows * nvec <= kResidentThreads) return go(I0{}, V1{});
   // two rows per wave where that keeps more lanes busy than one (the MoE
   // activation at I = 768 is 96 vectors, 75% of 64 x 2)
