@@ -582,39 +582,16 @@ int select_tile_cfg(int64_t M, int64_t N, int64_t K) {
   return cfg;
 }
 
-template <int BM, int BN, int KG, int WM, int WN, int KS, int NSTAGE, int EPI, int kWAux>
-int launch_ksplit_aux(const GemmArgs& g, unsigned blocks, hipStream_t st) {
-  using Sh = KsplitShape<BM, BN, KG, WM, WN, KS, NSTAGE>;
-  constexpr auto kern = ksplit_gemm_kernel<BM, BN, KG, WM, WN, KS, NSTAGE, EPI, kWAux>;
-  if (const int rc = set_lds_limit<kern>(Sh::kLds)) return rc;
-  hipLaunchKernelGGL(kern, dim3(blocks), dim3(Sh::kThreads), Sh::kLds, st, g);
-  return kOk;
-}
-
-// The weights stream with the non-temporal policy where every XCD's share of
-// the blocks is whole column ranges, so the row tiles of a range run side by
-// side on one XCD, for weights from kKsplitStreamBytes.  MI355X, weights from
-// HBM, default -> streaming, us: N 7168, K 5120 at M = 40 / 64 / 128 / 256
-// 13.3 / 14.3 / 18.7 / 23.7 -> 11.7 / 12.4 / 16.5 / 21.2; N 5120 at 64 / 128
-// / 256 13.6 / 16.9 / 20.8 -> 11.5 / 14.8 / 19.1; N 10240 at 64 / 128 25.0 /
-// 23.0 -> 22.1 / 21.0.  Not taken: three row tiles, whose ranges straddle
-// XCDs (N 7168, M = 333: 28.0 -> 28.5); the 128 x 128 tiles (M = 400 / 512:
-// 29.9 / 29.0 -> 30.7 / 29.4); weights of 10 - 13 MB, which the eight 4 MB
-// L2s hold (N 5120, K 2048 at 64 rows 7.4 -> 7.6; N 2560, K 5120 at 64 / 512
-// 10.2 / 18.7 -> 10.5 / 19.3).
-constexpr int64_t kKsplitStreamBytes = 20ll << 20;
-
 template <int BM, int BN, int KG, int WM, int WN, int KS, int NSTAGE, int EPI>
 int launch_ksplit(const GemmArgs& g, hipStream_t st) {
+  using Sh = KsplitShape<BM, BN, KG, WM, WN, KS, NSTAGE>;
+  constexpr auto kern = ksplit_gemm_kernel<BM, BN, KG, WM, WN, KS, NSTAGE, EPI>;
+  if (const int rc = set_lds_limit<kern>(Sh::kLds)) return rc;
   int64_t gm = 0;
   const int64_t gn = ksplit_ranges(g.M, g.N, KsplitCfg{BM, BN, KG, WM, WN, KS, NSTAGE}, gm);
   MW8_REQUIRE(gn > 0 && gm * gn < (int64_t{1} << 31), kErrShape, "gemm: no ksplit grid for N=%lld", (long long)g.N);
-  const unsigned blocks = static_cast<unsigned>(gm * gn);
-  if constexpr (EPI == kEpiBf16) {
-    if (BM * BN < 128 * 128 && (gn % kXcds == 0 || gm == 1) && g.N * g.K >= kKsplitStreamBytes)
-      return launch_ksplit_aux<BM, BN, KG, WM, WN, KS, NSTAGE, EPI, kStreamAux>(g, blocks, st);
-  }
-  return launch_ksplit_aux<BM, BN, KG, WM, WN, KS, NSTAGE, EPI, 0>(g, blocks, st);
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(gm * gn)), dim3(Sh::kThreads), Sh::kLds, st, g);
+  return kOk;
 }
 
 template <int EPI>

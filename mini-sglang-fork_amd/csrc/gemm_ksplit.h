@@ -90,10 +90,7 @@ struct KsplitShape {
   static_assert(kLds + 4 * (BM + 2 * BN) <= 163840, "LDS budget (ring or exchange + staging, scale tables)");
 };
 
-// kWAux: cache policy of the weight DMA.  kStreamAux where the row tiles that
-// share a weight range run side by side on one XCD (the host's rule): the
-// range is then fetched once either way, and does not evict the token rows.
-template <int BM, int BN, int KG, int WM, int WN, int KS, int NSTAGE, int EPI, int kWAux>
+template <int BM, int BN, int KG, int WM, int WN, int KS, int NSTAGE, int EPI>
 __global__ __launch_bounds__(64 * KG * WM * WN) void ksplit_gemm_kernel(GemmArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)
   using S = KsplitShape<BM, BN, KG, WM, WN, KS, NSTAGE>;
@@ -167,7 +164,7 @@ __global__ __launch_bounds__(64 * KG * WM * WN) void ksplit_gemm_kernel(GemmArgs
 #pragma unroll
     for (int j = 0; j < S::kLB; ++j) {
       const int d = wlds[j] < 0 ? NSTAGE * S::kStage : base + wlds[j];
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_ptr_t)(lds + d), 16, woff[j], k0, 0, kWAux);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_ptr_t)(lds + d), 16, woff[j], k0, 0, 0);
     }
   };
 
