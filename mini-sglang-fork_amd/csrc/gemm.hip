@@ -968,7 +968,7 @@ template <int BM, int BN, int BK, int WM, int WN, int NSTAGE, int EPI, int kPerC
 int launch_grouped_persist(const GemmArgs& g, hipStream_t st) {
   constexpr int kLds = NSTAGE * (BM + BN) * BK;
   constexpr auto kern =
-      grouped_persist_kernel<BM, BN, BK, WM, WN, NSTAGE, EPI, true, kPerCu, kAct, BK == 128 ? 16 : 32>;
+      grouped_persist_kernel<BM, BN, BK, WM, WN, NSTAGE, EPI, kPerCu, kAct, BK == 128 ? 16 : 32>;
   if (const int rc = set_lds_limit<kern>(kLds)) return rc;
   const unsigned grid = static_cast<unsigned>(device_cus() * kPerCu);
   hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * WM * WN), kLds, st, g);

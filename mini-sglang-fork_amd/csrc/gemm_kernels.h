@@ -77,8 +77,9 @@ struct GemmArgs {
   int32_t staged_out;
   // grouped GEMM over expert runs (SortedRunRows): rows of the alignment
   // blocks behind expert_ids / num_post_pad (the tile height BM is a
-  // multiple of it)
+  // multiple of it), and how many such blocks the lists have room for
   int32_t align_bsz;
+  int32_t align_blocks;
   // router-id rows (TopkRows): 16-pair units per expert (ceil(tokens / 16))
   int32_t topk_units;
 };
@@ -707,10 +708,9 @@ __device__ __forceinline__ void tile3_run(const GemmArgs& g, unsigned char* lds,
   for (int i = 0; i < kFM; ++i)
 #pragma unroll
     for (int j = 0; j < kFN; ++j) acc[i][j] = Acc{0};
-  // Run tiles: the sorted positions of a run are real pairs up to the
-  // expert's padding, which ends it, so the real rows of this wave's range
-  // form a prefix of length live_w; 32-row fragments past it (padding or
-  // past the run) have no MFMA work.  live_w is wave-uniform (ballot).
+  // Run tiles: the last real pair of this wave's row range ends at live_w
+  // (the expert's padding ends its run); fragments past it (padding or past
+  // the run) have no MFMA work.  live_w is wave-uniform (ballot).
   int live_w = kWaveM;
   if constexpr (Rows::kRuns) {
     live_w = 0;
@@ -718,7 +718,8 @@ __device__ __forceinline__ void tile3_run(const GemmArgs& g, unsigned char* lds,
     for (int h = 0; h < kWaveM; h += 64) {
       const int r = wm * kWaveM + h + lane;
       const bool real = h + lane < kWaveM && r < rows_valid && g.sorted_ids[m0 + r] < g.num_valid;
-      live_w += __popcll(__ballot(real));
+      const uint64_t rows = __ballot(real);
+      if (rows) live_w = h + 64 - __clzll(rows);
     }
     live_w = __builtin_amdgcn_readfirstlane(live_w);
   }
@@ -1165,18 +1166,18 @@ __global__ __launch_bounds__(64 * WM * WN) void tile3_gemm_kernel(GemmArgs g) {
 // Persistent grouped GEMM (fused-MoE, 64/128-row alignment blocks).
 // ------------------------------------------------------------------------
 // An expert's alignment blocks form ceil(blocks / per_tile) chunks of
-// near-equal size (per_tile = BM / align_bsz).  Work item = (expert with
-// at least one block, BN-column tile), the block running all its chunks in
-// turn (re-reading the weight tile it has just streamed), or, with
-// kChunkItems, (expert, column tile, chunk), the chunks of one weight tile
-// adjacent in the list and so running side by side on one XCD.
+// near-equal size (per_tile = BM / align_bsz).  Work item = (expert,
+// BN-column tile, chunk), the chunks of one weight tile adjacent in the list
+// and so running side by side on one XCD.
 // Every block derives the item list from expert_ids on its own (no
 // workspace, no extra launch): expert e's blocks are the run
-// [run_start[e], run_start[e + 1]) (expert_ids is non-decreasing over the
-// used blocks).  Items are numbered expert-major, and each XCD's blocks
-// (block b runs on XCD b % 8) deal one contiguous range of them, so all
-// column tiles of an expert share its gathered rows in one L2.  Each block
-// walks its items with a static stride: no queue, no inter-block waiting.
+// [run_start[e], run_start[e + 1]) where expert_ids is non-decreasing over
+// the used blocks, as the alignment writes it (a list in any other order is
+// walked block by block).  Items are numbered expert-major, and each XCD's
+// blocks (block b runs on XCD b % 8) deal one contiguous range of them, so
+// all column tiles of an expert share its gathered rows in one L2.  Each
+// block walks its items with a static stride: no queue, no inter-block
+// waiting.
 
 __device__ __forceinline__ int wave_incl_scan(int v) {
   const int lane = threadIdx.x & 63;
@@ -1190,32 +1191,45 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
 
 // Run tables of a grouped walk, built by every block from expert_ids:
 // run_start[e] = first alignment block of expert e (run_start[E] = blocks
-// in use) and act_base[e] = units (experts with blocks, or chunks of up to
-// per_tile blocks with kChunkItems) before e; returns the unit total.
+// in use) and act_base[e] = units (chunks of up to per_tile blocks) before
+// e; returns the unit total.
 // Ends with a __syncthreads: the tables are visible to the whole block.
-template <int kThreads, bool kChunkItems>
+//
+// The alignment lists the blocks by ascending expert, and the tables hold
+// for such lists.  A list in another order (or with ids outside [0, E)
+// between others) clears `runs`: then every alignment block in use is a unit
+// of its own, expert_ids names its expert, and the tables are not read.
+template <int kThreads>
 __device__ __forceinline__ int build_run_tables(const GemmArgs& g, int per_tile, int* run_start, int* act_base,
-                                                int* wave_tot) {
+                                                int* wave_tot, bool& runs) {
   constexpr int kWaves = kThreads / 64;
+  __shared__ int wave_steps_back[kWaves];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int E = g.num_experts, ab = g.align_bsz;
-  const int used = *g.num_post_pad / ab;  // alignment blocks in use
+  int used = (max(*g.num_post_pad, 0) + ab - 1) / ab;  // alignment blocks in use
+  if (used > g.align_blocks) used = g.align_blocks;
   // run starts: the block b where expert_ids steps from p to c starts the
   // runs of experts p+1 .. c (a virtual block `used` starts every later one)
+  bool back = false;
   for (int b = tid; b <= used; b += kThreads) {
-    const int prev = b == 0 ? -1 : g.expert_ids[b - 1];
-    int cur = b == used ? E : g.expert_ids[b];
-    if (cur > E) cur = E;
+    const int prev = b == 0 ? -1 : min(max(g.expert_ids[b - 1], -1), E);
+    const int cur = b == used ? E : min(g.expert_ids[b], E);
+    back |= cur < prev;
     for (int e = prev + 1; e <= cur; ++e) run_start[e] = b;
   }
+  const bool wave_back = __ballot(back) != 0;
+  if (lane == 0) wave_steps_back[wave] = wave_back;
   __syncthreads();
-  // exclusive prefix over experts of their unit count: 1 if the expert has
-  // blocks (expert items), or its chunk count (chunk items); two-level scan
+  int any_back = 0;
+  for (int w = 0; w < kWaves; ++w) any_back |= wave_steps_back[w];
+  runs = __builtin_amdgcn_readfirstlane(any_back) == 0;
+  if (!runs) return used;  // block-uniform
+  // exclusive prefix over experts of their chunk count; two-level scan
   int carry = 0;
   for (int e0 = 0; e0 < E; e0 += kThreads) {
     const int e = e0 + tid;
     const int len = e < E ? run_start[e + 1] - run_start[e] : 0;
-    const int act = kChunkItems ? (len + per_tile - 1) / per_tile : (len > 0 ? 1 : 0);
+    const int act = (len + per_tile - 1) / per_tile;
     const int incl = wave_incl_scan(act);
     if (lane == 63) wave_tot[wave] = incl;
     __syncthreads();
@@ -1232,8 +1246,7 @@ __device__ __forceinline__ int build_run_tables(const GemmArgs& g, int per_tile,
   return carry;
 }
 
-template <int BM, int BN, int BK, int WM, int WN, int NSTAGE, int EPI, bool kChunkItems, int kPerCu,
-          int kAct = -1, int MF = 32>
+template <int BM, int BN, int BK, int WM, int WN, int NSTAGE, int EPI, int kPerCu, int kAct = -1, int MF = 32>
 __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(kPerCu * WM * WN / 4)))
 void grouped_persist_kernel(GemmArgs g) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -1244,7 +1257,8 @@ void grouped_persist_kernel(GemmArgs g) {
   __shared__ int wave_tot[kWaves];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int E = g.num_experts, ab = g.align_bsz, per_tile = BM / ab;
-  const int carry = build_run_tables<kThreads, kChunkItems>(g, per_tile, run_start, act_base, wave_tot);
+  bool runs = true;
+  const int carry = build_run_tables<kThreads>(g, per_tile, run_start, act_base, wave_tot, runs);
   // column tiles: BN output columns, or BN / 2 activation columns (kAct)
   constexpr int kTileCols = kAct >= 0 ? BN / 2 : BN;
   const int64_t out_cols = kAct >= 0 ? g.N / 2 : g.N;
@@ -1257,41 +1271,42 @@ void grouped_persist_kernel(GemmArgs g) {
   const int begin = xcd * base + (xcd < rem ? xcd : rem), count = base + (xcd < rem ? 1 : 0);
   for (int j = local; j < count; j += per_xcd) {
     const int item = begin + j;
-    const int a = item / tn;  // expert items: the active-expert index
-    // the expert: last e with act_base[e] * tn <= item (act_base[e + 1] * tn > item)
-    int lo = 0, hi = E - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (act_base[mid] * tn <= item) lo = mid; else hi = mid - 1;
+    int e, c0, c1, n_tile;
+    if (runs) {
+      // the expert: last e with act_base[e] * tn <= item (act_base[e + 1] * tn > item)
+      int lo = 0, hi = E - 1;
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (act_base[mid] * tn <= item) lo = mid; else hi = mid - 1;
+      }
+      const int b_first = run_start[lo], nblocks = run_start[lo + 1] - b_first;
+      const int nch = (nblocks + per_tile - 1) / per_tile;
+      const int off = item - act_base[lo] * tn, c = off % nch;  // chunk fastest
+      e = lo;
+      n_tile = off / nch;
+      c0 = b_first + c * nblocks / nch;
+      c1 = b_first + (c + 1) * nblocks / nch;
+    } else {  // item = (alignment block, column tile)
+      c0 = item / tn;
+      e = g.expert_ids[c0];
+      n_tile = item - c0 * tn;
+      c1 = static_cast<unsigned>(e) < static_cast<unsigned>(E) ? c0 + 1 : c0;  // else nothing to compute
     }
-    const int e = __builtin_amdgcn_readfirstlane(lo);
-    const int b_first = __builtin_amdgcn_readfirstlane(run_start[e]);
-    const int nblocks = __builtin_amdgcn_readfirstlane(run_start[e + 1]) - b_first;
-    const int nch = (nblocks + per_tile - 1) / per_tile;
-    int n_tile, c_lo, c_hi;
-    if constexpr (kChunkItems) {  // item = (expert, column tile, chunk), chunk fastest
-      const int off = item - act_base[e] * tn;
-      n_tile = __builtin_amdgcn_readfirstlane(off / nch);
-      c_lo = __builtin_amdgcn_readfirstlane(off % nch);
-      c_hi = c_lo + 1;
-    } else {  // item = (expert, column tile): all chunks in turn
-      n_tile = __builtin_amdgcn_readfirstlane(item - a * tn);
-      c_lo = 0;
-      c_hi = nch;
-    }
-    for (int c = c_lo; c < c_hi; ++c) {
-      const int c0 = b_first + c * nblocks / nch, c1 = b_first + (c + 1) * nblocks / nch;
-      TileJob job{static_cast<int64_t>(c0) * ab,
-                  static_cast<int64_t>(n_tile) * kTileCols,
-                  g.W + static_cast<int64_t>(e) * g.N * g.K,
-                  g.sw + static_cast<int64_t>(e) * g.N,
-                  0,
-                  static_cast<int>(g.K / BK),
-                  (c1 - c0) * ab,
-                  -1};
-      __syncthreads();  // the previous tile's LDS staging has been read out
-      tile3_run<BM, BN, BK, WM, WN, NSTAGE, EPI, SortedRunRows, kAct, 0, MF>(g, lds, job);
-    }
+    e = __builtin_amdgcn_readfirstlane(e);
+    c0 = __builtin_amdgcn_readfirstlane(c0);
+    c1 = __builtin_amdgcn_readfirstlane(c1);
+    n_tile = __builtin_amdgcn_readfirstlane(n_tile);
+    if (c1 == c0) continue;  // block-uniform
+    TileJob job{static_cast<int64_t>(c0) * ab,
+                static_cast<int64_t>(n_tile) * kTileCols,
+                g.W + static_cast<int64_t>(e) * g.N * g.K,
+                g.sw + static_cast<int64_t>(e) * g.N,
+                0,
+                static_cast<int>(g.K / BK),
+                (c1 - c0) * ab,
+                -1};
+    __syncthreads();  // the previous tile's LDS staging has been read out
+    tile3_run<BM, BN, BK, WM, WN, NSTAGE, EPI, SortedRunRows, kAct, 0, MF>(g, lds, job);
   }
 #endif  // __HIP_DEVICE_COMPILE__
 }

@@ -115,7 +115,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void w
 
   // ---------------------------------------------------------------- walk
   const int per_tile = BM / g.align_bsz;
-  const int carry = build_run_tables<512, true>(g, per_tile, run_start, act_base, wave_tot);
+  bool runs = true;
+  const int carry = build_run_tables<512>(g, per_tile, run_start, act_base, wave_tot, runs);
   const int N32 = static_cast<int>(g.N), half32 = N32 / 2, K32 = static_cast<int>(g.K);
   const int lda32 = static_cast<int>(g.lda), ldo32 = static_cast<int>(g.ldo);
   const int nval32 = static_cast<int>(g.num_valid);
@@ -133,6 +134,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void w
     const int pos = local + j * per_xcd;
     if (pos >= count) return it;
     const int item = begin + pos;
+    it.ok = 1;
+    if (!runs) {  // a list that is not sorted by expert: (alignment block, column tile)
+      const int b = item / tn, e = g.expert_ids[b];
+      const bool real = static_cast<unsigned>(e) < static_cast<unsigned>(g.num_experts);
+      it.m0 = __builtin_amdgcn_readfirstlane(b * g.align_bsz);
+      it.n0 = __builtin_amdgcn_readfirstlane((item - b * tn) * kTileCols);
+      it.e = __builtin_amdgcn_readfirstlane(real ? e : 0);
+      it.rows = __builtin_amdgcn_readfirstlane(real ? g.align_bsz : 0);  // 0: nothing is written
+      return it;
+    }
     int lo = 0, hi = g.num_experts - 1;  // the expert: last e with act_base[e] * tn <= item
     while (lo < hi) {
       const int mid = (lo + hi + 1) >> 1;
@@ -146,7 +157,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void w
     it.n0 = __builtin_amdgcn_readfirstlane(n_tile * kTileCols);
     it.e = __builtin_amdgcn_readfirstlane(lo);
     it.rows = __builtin_amdgcn_readfirstlane((c1 - c0) * g.align_bsz);
-    it.ok = 1;
     return it;
   };
   // pair id of tile row r of an item whose sorted ids sit in t_p[par] (-1: padding or past the chunk)
@@ -387,11 +397,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void w
   for (;;) {
     const WalkItem nxt = item_of(jn++);
     int live;
-    {  // the chunk's pairs are a prefix of its rows: this wave's token fragments that hold pairs
-      int pairs = 0;
+    {  // this wave's token fragments up to the chunk's last pair
+      int end = 0;
 #pragma unroll
-      for (int h = 0; h < BM; h += 64) pairs += __popcll(__ballot(pair_of(par, h + opaque_lane(), cur.rows) >= 0));
-      const int frags = (pairs + MF - 1) / MF - wm;  // fragments wm, wm + 2, ... are this wave's
+      for (int h = 0; h < BM; h += 64) {
+        const uint64_t pairs = __ballot(pair_of(par, h + opaque_lane(), cur.rows) >= 0);
+        if (pairs) end = h + 64 - __clzll(pairs);
+      }
+      const int frags = (end + MF - 1) / MF - wm;  // fragments wm, wm + 2, ... are this wave's
       live = __builtin_amdgcn_readfirstlane(frags > 0 ? (frags + kWM - 1) / kWM : 0);
     }
 #pragma unroll

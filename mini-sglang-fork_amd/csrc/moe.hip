@@ -517,6 +517,7 @@ int moe_gemm_w8a8(const int8_t* A, const float* sa, const int8_t* W, const float
   g.topk_w = topk_w; g.num_valid = num_valid; g.top_k = top_k; g.num_experts = E;
   g.staged_out = epi == kEpiBf16 && N % 8 == 0 && aligned16(out);
   g.align_bsz = bsz;
+  g.align_blocks = static_cast<int32_t>(blocks);
   const int rc = bsz <= 32 ? launch_grouped_small(g, static_cast<unsigned>(blocks), epi, st)
                            : launch_grouped_tile(g, static_cast<unsigned>(blocks), bsz, epi, st);
   if (rc != kOk) return rc;
@@ -548,6 +549,7 @@ int moe_gemm_act_w8a8(const int8_t* A, const float* sa, const int8_t* W, const f
   g.topk_w = topk_w; g.num_valid = num_valid; g.top_k = top_k; g.num_experts = E;
   g.staged_out = 1;
   g.align_bsz = bsz;
+  g.align_blocks = static_cast<int32_t>(max_sorted / bsz);
   if (const int rc = launch_grouped_act(g, act, st)) return rc;
   return check_launch("moe_gemm_act");
 }

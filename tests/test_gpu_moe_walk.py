@@ -100,6 +100,88 @@ def test_walk_activation_equals_separate(act, routed):
     assert torch.equal(out.view(torch.int16), want.view(torch.int16))
 
 
+def _any_order(sorted_ids, expert_ids, npp, B, E, numel, seed):
+    """The same pairs in lists that the alignment would not write: blocks in
+    random order, padding between the pairs of a block, blocks of experts
+    outside [0, E) that name real pairs, a last block in use only in part and
+    room behind it."""
+    gen = torch.Generator().manual_seed(seed)
+    nb = int(npp.item()) // B
+    blocks, experts = sorted_ids[: nb * B].view(nb, B).cpu(), expert_ids[:nb].cpu()
+    few = (blocks < numel).sum(1).argmin()
+    last, last_e = blocks[few : few + 1], experts[few : few + 1]
+    keep = torch.arange(nb) != few
+    blocks, experts = blocks[keep], experts[keep]
+    blocks = blocks.gather(1, torch.rand(blocks.shape, generator=gen).argsort(1))
+    foreign = torch.arange(4 * B, dtype=torch.int32).view(4, B) % numel
+    blocks = torch.cat([blocks, foreign])
+    experts = torch.cat([experts, torch.tensor([-1, E, E + 7, -5], dtype=torch.int32)])
+    order = torch.randperm(len(experts), generator=gen)
+    blocks = torch.cat([blocks[order], last, torch.zeros(2, B, dtype=torch.int32)])
+    experts = torch.cat([experts[order], last_e, torch.zeros(2, dtype=torch.int32)])
+    used = (len(experts) - 3) * B + int((last < numel).sum())
+    return blocks.reshape(-1).to(DEV), experts.to(DEV), torch.tensor([used], dtype=torch.int32, device=DEV)
+
+
+@pytest.mark.parametrize("B", [64, 128])
+@pytest.mark.parametrize("few_pairs", [False, True])
+def test_lists_in_any_order(B, few_pairs):
+    """Lists whose blocks are not sorted by expert, in every configuration:
+    the grouped GEMM takes the expert of each alignment block from
+    expert_ids, whatever its neighbours are."""
+    k, N, K = 2, 512, 640
+    counts = [3, 0, 17, 2, 30, 1, 9, 0, 40, 5] if few_pairs else COUNTS
+    ids, W, SW, tw, gen = _case(counts, k, N, K, 21 + B)
+    M, E = ids.shape[0], W.shape[0]
+    idsd, twd, Wd, SWd = ids.to(DEV), tw.to(DEV), W.to(DEV), (SW * 1e-2).to(DEV)
+    aligned = moe_align_block_size(idsd, B, E)
+    lists = _any_order(*aligned, B, E, M * k, B)
+    q, s = quant_per_token(torch.randn(M, K, generator=gen).to(torch.bfloat16).to(DEV))
+    y_ref = orc.grouped_gemm_w8a8(q.cpu().numpy(), s.cpu().numpy(), W.numpy(), SWd.cpu().numpy(), ids.numpy(), k,
+                                  routed=tw.numpy())
+    lib = mw8lib.load()
+    try:
+        for cfg in (0, -1, 1, 2):
+            announce(f"any order B={B} few={few_pairs} cfg {cfg}")
+            lib.mw8_set_tuning(-1, -1, cfg)
+            out = torch.zeros(M * k, N, dtype=torch.bfloat16, device=DEV)
+            fused_moe_kernel_w8a8(q, s, Wd, SWd, out, twd, *lists, True, k, B, M * k)
+            torch.cuda.synchronize()
+            assert bf16_bits_equal(out, y_ref).all()
+        want = act_and_mul_quant(out, "silu", return_act=True)[2]
+        for cfg in (-1, 1, 2):
+            announce(f"any order B={B} few={few_pairs} activation cfg {cfg}")
+            lib.mw8_set_tuning(-1, -1, cfg)
+            act = torch.zeros(M * k, N // 2, dtype=torch.bfloat16, device=DEV)
+            fused_moe_kernel_act_w8a8(q, s, Wd, SWd, act, *lists, k, B, M * k, "silu", twd)
+            torch.cuda.synchronize()
+            assert torch.equal(act.view(torch.int16), want.view(torch.int16))
+    finally:
+        lib.mw8_set_tuning(-1, -1, -1)
+
+
+@pytest.mark.parametrize("used", [0, -64])
+def test_no_blocks_in_use(used):
+    """Nothing is written where num_post_pad says that no block is in use."""
+    ids, W, SW, tw, gen = _case([5, 3], 2, 256, 640, 4)
+    M, E = ids.shape[0], W.shape[0]
+    sorted_ids, expert_ids, npp = moe_align_block_size(ids.to(DEV), 64, E)
+    npp.fill_(used)
+    q, s = quant_per_token(torch.randn(M, 640, generator=gen).to(torch.bfloat16).to(DEV))
+    lib = mw8lib.load()
+    try:
+        for cfg in (0, 1, 2):
+            announce(f"no blocks in use: {used}, cfg {cfg}")
+            lib.mw8_set_tuning(-1, -1, cfg)
+            out = torch.full((M * 2, 256), 7, dtype=torch.bfloat16, device=DEV)
+            fused_moe_kernel_w8a8(q, s, W.to(DEV), SW.to(DEV), out, tw.to(DEV), sorted_ids, expert_ids, npp, False, 2,
+                                  64, M * 2)
+            torch.cuda.synchronize()
+            assert (out == 7).all()
+    finally:
+        lib.mw8_set_tuning(-1, -1, -1)
+
+
 def test_walk_preference_is_host_only():
     assert moe_gemm_act_preferred(2400, 1536, 2048, 128)
     assert not moe_gemm_act_preferred(100, 1536, 512, 128)  # four K stages: below the walk's fewest
