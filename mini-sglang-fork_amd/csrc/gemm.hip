@@ -360,7 +360,6 @@ constexpr KsplitCfg kKsplitCfgs[] = {
     {128, 128, 2, 2, 2, 2, 3, "ksplit_gemm_kernel<128, 128, 2, 2, 2, 2, 3>"},  // 4: 128-byte stages, 2 k-steps
 };
 constexpr int kNumKsplitCfgs = sizeof(kKsplitCfgs) / sizeof(kKsplitCfgs[0]);
-constexpr int kNumTileCfgs = kNumRingCfgs + kNumKsplitCfgs;
 
 // The 192 x 256 ring (8 waves 2x4 of 96 x 64, 2 A and 3 W slots with the
 // weight lead): three quarters of a 256 x 256 tile in three quarters of its
@@ -374,9 +373,10 @@ constexpr int kNumTileCfgs = kNumRingCfgs + kNumKsplitCfgs;
 // 256-row tiles fill whole waves it loses (4096 x 34816 x 5120 600 -> 646).
 // Its index follows the split-K tilings.
 constexpr TileCfg kRing192 = {192, 256, true, 128, 1, true, "tile3_gemm_kernel<192, 256, 128, 2, 4, 2>"};
-constexpr int kCfg192 = kNumTileCfgs;
+constexpr int kCfg192 = kNumRingCfgs + kNumKsplitCfgs;
+constexpr int kNumTileCfgs = kCfg192 + 1;
 
-constexpr bool is_ksplit(int cfg) { return cfg >= kNumRingCfgs && cfg < kNumTileCfgs; }
+constexpr bool is_ksplit(int cfg) { return cfg >= kNumRingCfgs && cfg < kCfg192; }
 constexpr const TileCfg& ring_cfg(int cfg) { return cfg == kCfg192 ? kRing192 : kTileCfgs[cfg]; }
 
 constexpr int ksplit_sk(const KsplitCfg& c) { return c.kg * c.ks * 32; }
@@ -569,7 +569,7 @@ int default_tile_cfg(int64_t M, int64_t N, int64_t K) {
 
 // The ring configuration a dense call at (M, N, K) runs (override first).
 bool tile_cfg_fits(int cfg, int64_t M, int64_t N, int64_t K) {
-  if (cfg < 0 || cfg > kCfg192) return false;
+  if (cfg < 0 || cfg >= kNumTileCfgs) return false;
   if (!is_ksplit(cfg)) return !ring_cfg(cfg).dma || K % ring_cfg(cfg).bk == 0;
   const KsplitCfg& c = kKsplitCfgs[cfg - kNumRingCfgs];
   int64_t gm = 0;
@@ -824,7 +824,9 @@ size_t gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 
 size_t gemm_workspace_max_bytes() {
   size_t mx = 0;
-  for (const TileCfg& c : kTileCfgs) {
+  for (int cfg = 0; cfg < kNumTileCfgs; ++cfg) {
+    if (is_ksplit(cfg)) continue;
+    const TileCfg& c = ring_cfg(cfg);
     if (!c.dma || !c.split) continue;
     const size_t b = static_cast<size_t>(device_cus()) * c.per_cu * c.bm * c.bn * sizeof(int32_t);
     if (b > mx) mx = b;

@@ -141,7 +141,7 @@ def test_workspace_bound_and_tuning_counts(lib):
     # the allocation-free entry's static scratch (64 MiB) holds every plan on 256 CUs
     assert mx <= 64 << 20
     counts = [lib.mw8_tuning_count(k) for k in range(4)]
-    assert counts == [10, 13, 3, 3] and lib.mw8_tuning_count(9) == 0
+    assert counts == [10, 14, 3, 3] and lib.mw8_tuning_count(9) == 0
     worst = 0
     try:
         for tile in range(-1, counts[1]):
@@ -152,6 +152,26 @@ def test_workspace_bound_and_tuning_counts(lib):
     finally:
         lib.mw8_set_tuning(-1, -1, -1)
     assert 0 < worst <= mx
+
+
+def test_tile_count_is_what_set_tuning_accepts(lib):
+    """Every tile index below the count selects a tiling of its own, and the
+    next one is no configuration: the automatic choice stays."""
+    M, N, K = 2080, 5120, 17408
+    auto = lib.mw8_gemm_kernel_name(M, N, K)
+    count = lib.mw8_tuning_count(1)
+    names = []
+    try:
+        for cfg in range(count):
+            lib.mw8_set_tuning(-1, cfg, -1)
+            names.append(lib.mw8_gemm_kernel_name(M, N, K))
+        assert len(set(names)) == count and auto in names
+        for cfg in (count, count + 1):
+            lib.mw8_set_tuning(-1, 2, -1)
+            lib.mw8_set_tuning(-1, cfg, -1)
+            assert lib.mw8_gemm_kernel_name(M, N, K) == auto
+    finally:
+        lib.mw8_set_tuning(-1, -1, -1)
 
 
 def test_linear_bf16_supported_shapes(lib):
