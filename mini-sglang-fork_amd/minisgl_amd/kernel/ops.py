@@ -20,9 +20,11 @@ _ACT = {"silu": 0, "gelu": 1}
 # The current stream's handle and the current device as integers, without
 # the Stream and device objects of torch.cuda.current_stream (1.9 us a call)
 # and torch.cuda.device (1.4 us): an eager decode call is a few launches of
-# 5-10 us each, and its host time is what bounds it.
-_raw_stream = torch._C._cuda_getCurrentRawStream
-_get_device = torch._C._cuda_getDevice
+# 5-10 us each, and its host time is what bounds it.  A torch built without
+# GPU support lacks both; the module then still loads, and a call raises on
+# its CPU tensors.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_get_device = getattr(torch._C, "_cuda_getDevice", None)
 
 
 def _stream(t: torch.Tensor) -> int:

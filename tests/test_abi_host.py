@@ -7,6 +7,8 @@ behaves like the reference.  No GPU compute happens here."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -14,6 +16,7 @@ import torch
 from minisgl_amd.kernel import lib as mw8lib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PKG_DIR = os.path.join(ROOT, "mini-sglang-fork_amd")
 HEADER = os.path.join(ROOT, "include", "mw8.h")
 CALIB_HEADER = os.path.join(ROOT, "include", "mw8_calib.h")
 
@@ -172,6 +175,26 @@ def test_tile_count_is_what_set_tuning_accepts(lib):
             assert lib.mw8_gemm_kernel_name(M, N, K) == auto
     finally:
         lib.mw8_set_tuning(-1, -1, -1)
+
+
+def test_wrappers_load_on_a_cpu_only_torch():
+    """A torch without GPU support lacks the bindings that name the current
+    stream and device: the package still imports, and a wrapper refuses CPU
+    tensors with its own error."""
+    code = (
+        "import sys, torch\n"
+        "for n in ('_cuda_getCurrentRawStream', '_cuda_getDevice'):\n"
+        "    delattr(torch._C, n)\n"
+        f"sys.path.insert(0, {PKG_DIR!r})\n"
+        "from minisgl_amd.kernel import quant_per_token\n"
+        "try:\n"
+        "    quant_per_token(torch.zeros(2, 8, dtype=torch.bfloat16))\n"
+        "except ValueError as e:\n"
+        "    assert 'GPU tensors' in str(e)\n"
+        "else:\n"
+        "    raise SystemExit('no error')\n"
+    )
+    subprocess.run([sys.executable, "-c", code], check=True, timeout=300)
 
 
 def test_linear_bf16_supported_shapes(lib):
