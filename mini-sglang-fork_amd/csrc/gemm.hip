@@ -1,6 +1,7 @@
 // Dense W8A8 GEMM: dispatch between the decode cores (M <= 32, or up to 64
 // when K % 128 != 0: weight streaming, in-block split-K) and the MFMA tile
 // ring, plus the grouped-tile launchers used by the fused-MoE GEMM.
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -1000,30 +1001,58 @@ int launch_walk(const GemmArgs& g, hipStream_t st) {
 // Grouped configurations for 64/128-row alignment blocks (mw8_set_tuning
 // moe_cfg): 0 one 128-wide ring tile per alignment block (tile height =
 // block size), 1 the persistent walk over (expert, column tile, chunk)
-// items with 128x256 tiles on 64-byte K stages, two blocks per CU.
+// items with 128x256 tiles on 64-byte K stages, two blocks per CU, 2 the
+// walk over tall items (gemm_walk.h), which takes whole 128-byte K stages
+// and whole column tiles (walk_fits; a call it does not take runs 0).
 //
-// 2 the walk over tall items (gemm_walk.h), which takes whole 128-byte K
-// stages and whole column tiles (walk_fits; else the automatic choice of 0
-// and 1).
-//
-// Automatic choice: the walk wherever it fits and the output is bf16.
-// Measured on MI355X (weights from HBM, us per launch, best of 0 and 1 ->
-// walk; GEMM1 with the activation in its epilogue / GEMM2): E 128, top-8,
-// H 2048, I 768 at 300 / 1024 / 2048 / 4096 / 8192 tokens GEMM1 79 / 85 /
-// 118 / 186 / 300 -> 67 / 72 / 80 / 146 / 236, GEMM2 45 / 59 / 86 / 129 /
-// 218 -> 43 / 52 / 65 / 114 / 193; E 64, top-6, H 4096, I 1152 at 4096
-// tokens 333 / 219 -> 250 / 188; E 16, top-2, H 4096, I 1408 at 2500 tokens
-// 106 / 51 -> 81 / 46.  Where it does not fit: with at least 32 pairs per
-// expert on average the persistent chunk walk (cfg 1): 1024 tokens 237 ->
-// 215 us per layer, 4096 tokens 536 -> 459 us against cfg 0; at 16 pairs per
-// expert (256 tokens) cfg 0 (167 us against 177).
+// Without the tall walk: with at least 32 pairs per expert on average the
+// persistent chunk walk (E 128, top-8, H 2048, I 768, us per layer, 0 -> 1:
+// 1024 tokens 237 -> 215, 4096 tokens 536 -> 459), else 0 (256 tokens, 16
+// pairs per expert: 167 against 177).
 constexpr int kNumMoeCfgs = 3;
+constexpr int64_t kPersistMinPairs = 32;  // pairs per expert
+bool persist_pays(int64_t num_valid, int64_t E) { return num_valid >= kPersistMinPairs * E; }
+
+// Whether the tall walk is faster than that choice.  Its time is a number of
+// rounds of one item (192 rows x 256 weight rows of the whole K) per CU, so
+// the items decide, counted here for pairs spread over the experts.  Measured
+// on MI355X over 3550 random layers (E 4-256, top 2-8, H 768-5120, I 256-2048,
+// up to 8192 tokens; weights from HBM; walk against the choice above, GEMM1 /
+// GEMM2 medians): where this rule takes it 0.87 / 0.87 of the time, where it
+// does not 1.08 / 1.14; 0.7% / 0.5% of the calls are more than 3% slower for
+// it.  us, the choice above -> walk:
+//  * below 32 pairs per expert the tiles (64 x 128) put up to 6 blocks on the
+//    CUs for each item: E 8, H 2048, I 768, 40 tokens 13.6 -> 20.9 (48 items),
+//    E 32, H 1024, I 1408, 40 tokens, GEMM2 13.3 -> 16.0 (128 items), E 16, H
+//    1024, I 1408 18.5 -> 17.1 (176 items).  With few K stages the walk's
+//    start and end weigh more: K 768, 160 items 10.5 -> 13.6;
+//  * a second round that few blocks run: E 32, H 1024, I 1408, 40 tokens 24.3
+//    -> 26.6 (352 items), E 16, H 1536, K 896, 609 pairs per expert 29.4 ->
+//    37.5; also a third one, and two whole rounds on rows of 4096 bytes (E 64,
+//    N 2048, K 4096 107 -> 117);
+//  * full chunks of few K stages, where the epilogue is a third of an item:
+//    E 16, N 2048, K 640, 1975 pairs per expert 81.5 -> 108.3; K 768, 4958
+//    pairs 112 -> 137.
+bool walk_pays(int64_t num_valid, int64_t N, int64_t K, int64_t E, int align_bsz, bool act) {
+  const double cus = device_cus(), pairs = static_cast<double>(num_valid) / static_cast<double>(E);
+  const int rows = kWalkBM / align_bsz * align_bsz;  // of a full chunk
+  // chunks: one per expert, or pairs / rows and half a chunk for the last
+  const bool spread = pairs >= 160.0;  // the experts' chunk counts differ
+  const double chunks = spread ? static_cast<double>(E) * std::max(1.0, pairs / rows + 0.5)
+                               : static_cast<double>(std::min(E, num_valid));
+  const double rounds = chunks * static_cast<double>(N / kWalkBN) / cus;
+  const bool few_pairs = !persist_pays(num_valid, E);
+  if (few_pairs && rounds < (K < 1024 ? 0.875 : 0.5625)) return false;
+  if (few_pairs && K % 4096 == 0 && rounds >= 1.0 && rounds < 2.35) return false;
+  if (rounds > (spread ? 0.9 : 1.0) && rounds < (few_pairs ? 1.56 : spread ? 1.625 : 1.375)) return false;
+  if (rounds > 2.0 && rounds < 2.35) return false;
+  if (pairs >= 512 && K < 1024) return false;
+  return act || pairs < 1000 || K >= 1536;
+}
+
 int default_moe_cfg(const GemmArgs& g, int epi) {
-  if (epi == kEpiBf16 && walk_fits(g)) return 2;
-  if (g.K % 64 == 0 && g.num_experts < kPersistMaxSlots &&
-      g.num_valid >= 32 * static_cast<int64_t>(g.num_experts))
-    return 1;
-  return 0;
+  if (epi == kEpiBf16 && walk_fits(g) && walk_pays(g.num_valid, g.N, g.K, g.num_experts, g.align_bsz, false)) return 2;
+  return g.num_experts < kPersistMaxSlots && persist_pays(g.num_valid, g.num_experts) ? 1 : 0;
 }
 
 template <int EPI>
@@ -1168,25 +1197,31 @@ int launch_moe_gemm_sum(const GemmArgs& g, int64_t max_sorted, hipStream_t st, b
   return kOk;
 }
 
-// Gate|up GEMM with the gated activation fused (the grouped walk, or the
-// persistent chunk walk where it does not fit or moe cfg 0 or 1 is forced):
-// out [rows, N/2] = act(gate) * up, bf16.
+// Gate|up GEMM with the gated activation fused: out [rows, N/2] = act(gate) *
+// up, bf16.  The tall walk where it fits and is the faster one (below 32
+// pairs per expert always: E 8, H 1024, I 768, 12 tokens 16.8 -> 15.4 us), or
+// the persistent chunk walk; moe cfg 0 and 1 force the latter.
 int launch_grouped_act(const GemmArgs& g, int act, hipStream_t st) {
   const int cfg = g_moe_cfg;
-  if ((cfg < 0 || cfg >= 2) && walk_fits(g)) return act == 0 ? launch_walk<0>(g, st) : launch_walk<1>(g, st);
+  const bool walk = cfg == 2 || ((cfg < 0 || cfg >= kNumMoeCfgs) &&
+                                 (!persist_pays(g.num_valid, g.num_experts) ||
+                                  walk_pays(g.num_valid, g.N, g.K, g.num_experts, g.align_bsz, true)));
+  if (walk && walk_fits(g)) return act == 0 ? launch_walk<0>(g, st) : launch_walk<1>(g, st);
   if (act == 0) return launch_grouped_persist<128, 256, 64, 2, 2, 3, kEpiBf16, 2, 0>(g, st);
   return launch_grouped_persist<128, 256, 64, 2, 2, 3, kEpiBf16, 2, 1>(g, st);
 }
 
 // Whether the fused-activation GEMM1 is the faster first step of a prefill
-// MoE layer (64/128-row alignment blocks; w1 [E, N = 2I, K]): wherever the
-// grouped walk takes it (300 tokens at E 128, top-8, H 2048, I 768: 79 us and
-// a 5.6 us activation kernel -> 67 us and a 4 us quantizer), else from 32
-// pairs per expert (the persistent chunk walk's range).
+// MoE layer (64-row alignment blocks; w1 [E, N = 2I, K]): from 32 pairs per
+// expert, and below where the tall walk beats the tiles and an activation
+// kernel (300 tokens at E 128, top-8, H 2048, I 768: 79 us and 5.6 us -> 67 us
+// and a 4 us quantizer).
 int moe_gemm_act_preferred(int64_t num_valid, int64_t N, int64_t K, int E) {
   if (num_valid < 0 || N <= 0 || N % 16 != 0 || K <= 0 || K % 64 != 0 || E < 1 || E >= kPersistMaxSlots) return 0;
-  if ((g_moe_cfg < 0 || g_moe_cfg >= 2) && walk_takes(N, K, E, num_valid, N / 2)) return 1;
-  return num_valid >= 32 * static_cast<int64_t>(E) ? 1 : 0;
+  if (persist_pays(num_valid, E)) return 1;
+  if (!walk_takes(N, K, E, num_valid, N / 2)) return 0;
+  if (g_moe_cfg == 2) return 1;
+  return (g_moe_cfg < 0 || g_moe_cfg >= kNumMoeCfgs) && walk_pays(num_valid, N, K, E, 64, true) ? 1 : 0;
 }
 
 }  // namespace mw8

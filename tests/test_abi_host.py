@@ -177,6 +177,18 @@ def test_tile_count_is_what_set_tuning_accepts(lib):
         lib.mw8_set_tuning(-1, -1, -1)
 
 
+def test_few_walk_items_stay_on_the_tiles(lib):
+    """A prefill MoE layer whose tall-walk items are too few for the CUs, or
+    leave a second round that few blocks run, keeps the tiles and a separate
+    activation (sizes where the walk measured 9-56% slower); where the items
+    fill the CUs the walk's fused activation is preferred."""
+    pref = lambda tokens, k, E, H, I: lib.mw8_moe_gemm_act_preferred(tokens * k, 2 * I, H, E)  # noqa: E731
+    for c in [(40, 2, 8, 2048, 768), (12, 4, 8, 1024, 1408), (130, 2, 16, 1024, 256), (40, 2, 32, 1024, 1408)]:
+        assert pref(*c) == 0, c
+    for c in [(130, 2, 16, 1024, 1408), (300, 8, 128, 2048, 768), (4096, 8, 128, 2048, 768)]:
+        assert pref(*c) == 1, c
+
+
 def test_wrappers_load_on_a_cpu_only_torch():
     """A torch without GPU support lacks the bindings that name the current
     stream and device: the package still imports, and a wrapper refuses CPU

@@ -187,3 +187,28 @@ def test_walk_preference_is_host_only():
     assert not moe_gemm_act_preferred(100, 1536, 512, 128)  # four K stages: below the walk's fewest
     assert moe_gemm_act_preferred(32 * 128, 1536, 512, 128)
     assert not moe_gemm_act_preferred(2400, 1536, 2040, 128)
+
+
+@pytest.mark.parametrize("tokens,top_k,E,H,I", [(12, 4, 8, 1024, 768), (40, 2, 32, 1024, 1408), (130, 2, 16, 1024, 1408),
+                                                (700, 2, 8, 1024, 768), (4000, 2, 8, 256, 640)])
+def test_layer_equals_forced_tiles(tokens, top_k, E, H, I):
+    """A layer on each side of the choice between the tiles, the chunk walk
+    and the tall walk: the bits of the tiles."""
+    from minisgl_amd.moe.fused import fused_experts_impl_w8a8
+
+    announce(f"walk choice T={tokens} k={top_k} E={E} H={H} I={I}")
+    gen = torch.Generator().manual_seed(tokens + E)
+    w1 = torch.randint(-127, 128, (E, 2 * I, H), generator=gen, dtype=torch.int8).to(DEV)
+    w2 = torch.randint(-127, 128, (E, H, I), generator=gen, dtype=torch.int8).to(DEV)
+    s1, s2 = (torch.rand(E, n, generator=gen).to(DEV) * 1e-3 for n in (2 * I, H))
+    x = torch.randn(tokens, H, generator=gen).to(torch.bfloat16).to(DEV)
+    ids = torch.rand(tokens, E, generator=gen).topk(top_k, dim=1).indices.int().to(DEV)
+    tw = torch.rand(tokens, top_k, generator=gen).to(DEV)
+    lib = mw8lib.load()
+    got = fused_experts_impl_w8a8(x.clone(), w1, s1, w2, s2, tw, ids)
+    try:
+        lib.mw8_set_tuning(-1, -1, 0)
+        want = fused_experts_impl_w8a8(x.clone(), w1, s1, w2, s2, tw, ids)
+    finally:
+        lib.mw8_set_tuning(-1, -1, -1)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
