@@ -415,6 +415,9 @@ bool dispatch_rows(int64_t nvec, int64_t rows, hipStream_t st, Args... args) {
   if (nvec <= 32) return go(I32{}, V1{});
   if (nvec <= 64) return go(I64{}, V1{});
   if (nvec > 1024) {
+    // a launch holds fewer than 2^32 threads: 8 vectors each keep the blocks
+    // at 256 threads where that many rows fit the memory
+    if (rows >= (int64_t{1} << 23)) return go(I0{}, V8{});
     if (rows <= 512) return go(I0{}, V4{});
     if (nvec <= 512 * 3) return go(I0{}, V3{});
     if (nvec <= 512 * 5) return go(I0{}, V5{});
