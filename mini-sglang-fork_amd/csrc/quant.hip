@@ -19,6 +19,9 @@
 #include "mw8_common.h"
 
 namespace mw8 {
+
+int device_cus();
+
 namespace {
 
 constexpr int kBlock = 256;
@@ -365,30 +368,62 @@ __global__ __launch_bounds__(TPR > 0 ? kBlock : 64 * kMaxWaves) void rmsnorm_row
 
 // Pick (TPR, VPT) for rows of nvec 16-byte vectors; false if none fits.
 //
-// Measured on MI355X (graph nodes of 10 rotating inputs, us; the earlier
-// choice of 64 threads up to 512 vectors and 256 above -> this one).  Where
-// one thread per vector fits the chip's 512 Ki resident threads, every load
-// is in flight at once and the row's serial part (reductions, the quotient,
-// the activation) is shortest: quant 512 x 5120 5.1 -> 4.8, 777 x 3072 6.2
-// -> 4.8; gelu 777 x 3072 12.3 -> 7.6; silu 16 x 3072 7.2 -> 4.0, 2400 x
-// 768 5.8 -> 5.4; norm 300 x 2048 4.5 -> 3.8.  Longer rows take the fewest
-// vectors that 1024 threads hold (silu 64 x 17408 9.0 -> 7.1, quant 6.2 ->
-// 4.9 at one row), and past 512 rows 3, 5, 7 or 8 in blocks of up to 512
-// threads: quant 2080 x 25600 39.2 -> 33.2 (7; blocks of 256 x 16 left 32
-// rows to a round of their own), 5000 x 25600 76.7 -> 68.6, 8192 x 17408 77.2
-// -> 75.4 (5; 3, 4, 6, 7 80.4, 77.4, 77.0, 79.0), 8192 x 12288 53.0 -> 50.6
-// (3; 5 53.6).  Rows of 513 - 1024 vectors beyond the
-// resident threads: 6 per thread (quant 2080 x 6400 11.7 -> 10.1, norm 2080
-// x 5120 14.0 -> 12.7; one per thread 11.4 against 9.5 for 2080 x 5120), 3
-// or 4 from 4096 rows (norm + residual 8192 x 5120 53.6 against 56.5 with
-// 6, quant 6000 x 8192 28.2 with 4 against 29.4 with 3).
-// Up to 16 vectors four rows share a wave: the per-head norms (H = 128),
-// which kept 16 lanes of a wave busy, 2080 x 64 heads 46.2 -> 16.3 and 512 x
-// 40 heads 10.0 -> 4.8.
-constexpr int64_t kResidentThreads = 512 * 1024;
+// Up to 64 vectors (512 elements) a row takes 16, 32 or 64 lanes, one vector
+// each (the per-head norms of H = 128: 2080 x 64 heads 46.2 us on a wave per
+// row -> 16.3).  Longer rows get a block each.  The fewest vectors per thread
+// (1-9) with which the blocks of all rows are resident at once are the
+// fastest: every load is in flight together, and the row's serial part
+// (reductions, the quotient, the activation) is shortest.  With fewer, a few
+// blocks run a round of their own: quant 1110 x 17408 12.9 us with 7 vectors,
+// 15.6 with 5 (1024 rows resident), 1500 x 5120 7.0 with 3, 8.1 with 6.
+//
+// Rows that are not resident at once stream.  Then 129 - 512 vectors run one
+// row per wave, and longer rows 3 (up to 768 vectors), 4 (up to 1024) or as
+// many vectors as blocks of 512 threads hold (quant 8192 x 17408 75.4 us with
+// 5; 3, 4, 6, 7 80.4, 77.4, 77.0, 79.0).  The activation and the quantizing
+// norm compute more per vector and want more threads: from 193 to 1024
+// vectors 2 per thread (norm + residual 8192 x 4096 51.8 us on a wave per row
+// -> 43.6, 8192 x 5120 53.6 with 3 -> 52.8), residency with at most 5 and 4,
+// and past 768 vectors (12 waves) the norm never 1 (1 x 8192 5.2 us, with 2
+// 4.8; 1 x 6144 4.4 and 4.6).
+// Rows of 65 - 128 vectors: blocks up to 3072 rows (plain norm 2304, with the
+// quantizer 1024), then wave rows, two to a wave up to 96 vectors (act 8192 x
+// 768 9.7 us on one -> 8.9; the norms from 4096 rows).
+//
+// MI355X, graph nodes of 10 rotating inputs, 1436 combinations of operation,
+// 64 - 8192 rows and 65 - 4096 vectors: 1% off the fastest layout on average.
+enum class RowWork { kQuant, kAct, kNorm, kNormQuant };
+
+// Rows whose blocks of `waves` waves are resident at once.  A CU has 4 x 8
+// wave slots, which blocks of a multiple of 4 waves fill; others pack worse
+// (10 waves: two blocks, not three; 5: some of the time five, counted only
+// if `loose`).  Blocks of one or two waves slow down before the slots are
+// full (quant 4096 x 2048, 2 waves, 7.8 us; on wave rows 7.5), the quantizing
+// norm's of three as well.  The activation and that norm run blocks of 10
+// waves and more one to a CU (act 420 x 16384 10.0 us with 16 waves, 9.7 with
+// 8; 420 x 20480 11.3 with 14 or 8, 12.3 with 10).
+inline bool heavy_rows(RowWork work) { return work == RowWork::kAct || work == RowWork::kNormQuant; }
+
+inline int64_t resident_rows(RowWork work, int64_t waves, bool loose) {
+  if (waves > kMaxWaves) return 0;
+  int64_t per_cu = waves % 4 == 0 || waves < 4 ? 32 / waves : 29 / waves;
+  if (waves == 5 || waves == 6) per_cu = loose ? 5 : 4;
+  if (waves >= 10 && heavy_rows(work)) per_cu = 1;
+  const int64_t rows = per_cu * device_cus();
+  return waves < 3 || (waves == 3 && work == RowWork::kNormQuant) ? rows * 3 / 4 : rows;
+}
+
+// The fewest vectors per thread, from `least` to `most`, of block rows whose
+// blocks are resident at once; 0: none.
+inline int resident_vectors(RowWork work, int64_t nvec, int64_t rows, int least, int most) {
+  for (const bool loose : {false, true})
+    for (int v = least; v <= most; ++v)
+      if (resident_rows(work, (nvec + 64 * v - 1) / (64 * v), loose) >= rows) return v;
+  return 0;
+}
 
 template <template <int, int> class Launch, typename... Args>
-bool dispatch_rows(int64_t nvec, int64_t rows, hipStream_t st, Args... args) {
+bool dispatch_rows(RowWork work, int64_t nvec, int64_t rows, hipStream_t st, Args... args) {
   auto go = [&](auto tpr_c, auto vpt_c) {
     constexpr int TPR = decltype(tpr_c)::value;
     constexpr int VPT = decltype(vpt_c)::value;
@@ -410,30 +445,49 @@ bool dispatch_rows(int64_t nvec, int64_t rows, hipStream_t st, Args... args) {
   using V6 = std::integral_constant<int, 6>;
   using V7 = std::integral_constant<int, 7>;
   using V8 = std::integral_constant<int, 8>;
+  using V9 = std::integral_constant<int, 9>;
+  auto block_rows = [&](int v) {
+    switch (v) {
+      case 1: return go(I0{}, V1{});
+      case 2: return go(I0{}, V2{});
+      case 3: return go(I0{}, V3{});
+      case 4: return go(I0{}, V4{});
+      case 5: return go(I0{}, V5{});
+      case 6: return go(I0{}, V6{});
+      case 7: return go(I0{}, V7{});
+      case 8: return go(I0{}, V8{});
+      default: return go(I0{}, V9{});
+    }
+  };
+  auto wave_rows = [&] {  // two rows per wave, or one
+    const bool norm = work == RowWork::kNorm || work == RowWork::kNormQuant;
+    if (nvec <= 96 && (!norm || rows > 4096)) return go(I32{}, V3{});
+    if (nvec <= 64 * 2) return go(I64{}, V2{});
+    if (nvec <= 64 * 3) return go(I64{}, V3{});
+    if (nvec <= 64 * 4) return go(I64{}, V4{});
+    return nvec <= 64 * 6 ? go(I64{}, V6{}) : go(I64{}, V8{});
+  };
   if (nvec > 1024 * 4) return false;  // 32768 elements
   if (nvec <= 16) return go(I16{}, V1{});
   if (nvec <= 32) return go(I32{}, V1{});
   if (nvec <= 64) return go(I64{}, V1{});
-  if (nvec > 1024) {
-    // a launch holds fewer than 2^32 threads: 8 vectors each keep the blocks
-    // at 256 threads where that many rows fit the memory
-    if (rows >= (int64_t{1} << 23)) return go(I0{}, V8{});
-    if (rows <= 512) return go(I0{}, V4{});
-    if (nvec <= 512 * 3) return go(I0{}, V3{});
-    if (nvec <= 512 * 5) return go(I0{}, V5{});
-    return nvec <= 512 * 7 ? go(I0{}, V7{}) : go(I0{}, V8{});
+  // a launch holds fewer than 2^32 threads: small blocks for rows by the million
+  if (rows >= (int64_t{1} << 23)) return nvec <= 512 ? wave_rows() : block_rows(9);
+  const bool heavy = heavy_rows(work);
+  if (nvec <= 128) {
+    const int64_t most = work == RowWork::kNormQuant ? 1024 : work == RowWork::kNorm ? 2304 : 3072;
+    return rows <= most ? block_rows(1) : wave_rows();
   }
-  if (rows * nvec <= kResidentThreads) return go(I0{}, V1{});
-  // two rows per wave where that keeps more lanes busy than one (the MoE
-  // activation at I = 768 is 96 vectors, 75% of 64 x 2)
-  if (nvec <= 96) return go(I32{}, V3{});
-  if (nvec <= 64 * 2) return go(I64{}, V2{});
-  if (nvec <= 64 * 3) return go(I64{}, V3{});
-  if (nvec <= 64 * 4) return go(I64{}, V4{});
-  if (nvec <= 64 * 6) return go(I64{}, V6{});
-  if (nvec <= 64 * 8) return go(I64{}, V8{});
-  if (rows < 4096) return go(I0{}, V6{});
-  return nvec <= 768 ? go(I0{}, V3{}) : go(I0{}, V4{});  // up to 256 threads
+  if (nvec <= 512) {
+    // blocks of one wave would be wave rows
+    if (const int v = resident_vectors(work, nvec, rows, 1, nvec <= 192 ? 2 : 3)) return block_rows(v);
+    return heavy && nvec > 192 ? block_rows(2) : wave_rows();
+  }
+  const int least = work == RowWork::kNormQuant && nvec > 768 ? 2 : 1;
+  const int most = work == RowWork::kNormQuant ? 4 : work == RowWork::kAct ? 5 : 9;
+  if (const int v = resident_vectors(work, nvec, rows, least, most)) return block_rows(v);
+  if (nvec <= 1024) return block_rows(heavy ? 2 : nvec <= 768 ? 3 : 4);
+  return block_rows(static_cast<int>((nvec + 511) / 512));
 }
 
 template <int TPR, int VPT>
@@ -494,7 +548,7 @@ int quant_per_token_bf16(const void* x, int64_t M, int64_t K, int64_t ldx, int8_
   const auto* xb = static_cast<const uint16_t*>(x);
   const bool vec_ok = (K % 8 == 0) && (ldx % 8 == 0) && (ldq % 8 == 0) && aligned16(x) &&
                       aligned8(q);
-  if (!(vec_ok && dispatch_rows<QuantLaunch>(K / 8, M, st, xb, ldx, M, K, q, ldq, s))) {
+  if (!(vec_ok && dispatch_rows<QuantLaunch>(RowWork::kQuant, K / 8, M, st, xb, ldx, M, K, q, ldq, s))) {
     hipLaunchKernelGGL(quant_rows_generic_kernel, dim3(static_cast<unsigned>(M)), dim3(kBlock), 0,
                        st, xb, ldx, M, K, q, ldq, s);
   }
@@ -513,7 +567,7 @@ int act_and_mul_quant_bf16(const void* x, int64_t R, int64_t two_d, int act, int
   MW8_REQUIRE(aligned16(x) && aligned8(q) && (!a_out || aligned16(a_out)), kErrAlign,
               "act_and_mul_quant: x/act_out need 16-byte and q 8-byte alignment");
   const int64_t d = two_d / 2;
-  const bool ok = dispatch_rows<ActLaunch>(d / 8, R, st, static_cast<const uint16_t*>(x), R, d, act,
+  const bool ok = dispatch_rows<ActLaunch>(RowWork::kAct, d / 8, R, st, static_cast<const uint16_t*>(x), R, d, act,
                                            q, s, static_cast<uint16_t*>(a_out));
   MW8_REQUIRE(ok, kErrShape, "act_and_mul_quant: d=%lld exceeds the register-resident limit 32768",
               (long long)d);
@@ -533,8 +587,8 @@ int rmsnorm_quant_bf16(const void* x, void* residual, const void* weight, float 
   MW8_REQUIRE(aligned16(x) && aligned16(weight) && (!q || aligned8(q)) && (!residual || aligned16(residual)) &&
                   (!y || aligned16(y)),
               kErrAlign, "rmsnorm_quant: x/residual/weight/y need 16-byte and q 8-byte alignment");
-  const bool ok = dispatch_rows<NormLaunch>(H / 8, M, st, static_cast<const uint16_t*>(x),
-                                            static_cast<uint16_t*>(residual),
+  const bool ok = dispatch_rows<NormLaunch>(q ? RowWork::kNormQuant : RowWork::kNorm, H / 8, M, st,
+                                            static_cast<const uint16_t*>(x), static_cast<uint16_t*>(residual),
                                             static_cast<const uint16_t*>(weight), eps, M, H, q, s,
                                             static_cast<uint16_t*>(y), int64_t{1}, H, H);
   MW8_REQUIRE(ok, kErrShape, "rmsnorm_quant: H=%lld exceeds the register-resident limit 32768",
@@ -557,7 +611,7 @@ int rmsnorm_strided_bf16(const void* x, int64_t ldx, void* y, int64_t ldy, const
   MW8_REQUIRE(M < (1ll << 31) && M / inner == G, kErrShape, "rmsnorm_strided: too many rows");
   MW8_REQUIRE(aligned16(x) && aligned16(y) && aligned16(weight), kErrAlign,
               "rmsnorm_strided: x, y and weight need 16-byte alignment");
-  const bool ok = dispatch_rows<NormLaunch>(H / 8, M, st, static_cast<const uint16_t*>(x),
+  const bool ok = dispatch_rows<NormLaunch>(RowWork::kNorm, H / 8, M, st, static_cast<const uint16_t*>(x),
                                             static_cast<uint16_t*>(nullptr),
                                             static_cast<const uint16_t*>(weight), eps, M, H,
                                             static_cast<int8_t*>(nullptr), static_cast<float*>(nullptr),
