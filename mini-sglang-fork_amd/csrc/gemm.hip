@@ -540,6 +540,33 @@ int default_ksplit_cfg(int64_t M, int64_t N, int64_t K) {
 // -> 1228, down M=8192 591 -> 635, qkv M=8192 263 -> 283).
 constexpr int64_t kStreamMaxStages = 15;
 
+// Whether the 192 x 256 ring, whose modelled time `us` is below `best_us` of
+// configuration `best`, is taken.  The model misses where (MI355X, 1046 random
+// shapes where it preferred this ring, weights from HBM; earlier choice -> 192
+// x 256, us; refused: 1.00 - 1.11 of the time, taken: 0.87 - 0.97, one shape
+// 4% slower):
+//  * every tile would split along K: the other tilings' splits are as fast or
+//    faster (800 x 5120 x 17408 103 -> 109, 1024 x 5120 x 25600 144 -> 159);
+//  * a last wave split along K, unless it stands against 256 x 320, follows
+//    one whole wave and is a sixteenth of one (34816 columns, 257 - 384 rows:
+//    x 8192 138 -> 117): 822 x 17408 x 17408 255 -> 277 (84 tiles in 3 ranges),
+//    3428 x 8192 x 25600 607 -> 685 (64 in 4), 7475 x 5120 x 17408 514 -> 539
+//    (12 behind three waves), 6403 x 2048 x 25600 against 256 x 256 287 -> 328;
+//    with a seventh less modelled time it wins (566 x 25600 x 17408 288 -> 254);
+//  * 128-column tiles re-read weights of 250 MB and more, past the 256 MB
+//    cache: 435 x 17408 x 25600 255 -> 299, 2131 x 10240 x 25600 548 -> 574;
+//  * against 128 x 128, two per CU, on a part-filled chip, which the model
+//    rates too low (301 x 17408 x 25600 216 -> 286, 574 x 12800 x 17408 156 ->
+//    168), and with fewer than five K stages (1629 x 12240 x 512 27 -> 32).
+bool ring192_pays(int64_t M, int64_t N, int64_t K, double us, int best, double best_us) {
+  const SplitPlan sp = plan_split(M, N, K, kRing192);
+  if (sp.sp > 1 && sp.full == 0) return false;
+  if (sp.sp > 1 && (best != 6 || sp.sp < 16 || sp.full > device_cus()) && us > 0.87 * best_us) return false;
+  const bool narrow = best == 1 || best == 3 || best == 4;
+  if (narrow && N * K >= 250000000) return false;
+  return best == 3 || !narrow || (us <= 0.97 * best_us && K >= 640);
+}
+
 int default_tile_cfg(int64_t M, int64_t N, int64_t K) {
   if (K % 64 != 0) return 0;
   const int ks = default_ksplit_cfg(M, N, K);
@@ -548,18 +575,16 @@ int default_tile_cfg(int64_t M, int64_t N, int64_t K) {
   double best_us = 1e300;
   for (const ModelCfg& mc : kModelCfgs) {
     if (K % ring_cfg(mc.cfg).bk != 0) continue;
-    if (mc.cfg == kCfg192) {
-      // not where every tile would split along K: the other tilings' splits
-      // are as fast or faster (800 x 5120 x 17408 109 against 103 us, 1024 x
-      // 5120 x 25600 159 against 144, 512 x 5120 x 17408 level)
-      const SplitPlan sp = plan_split(M, N, K, kRing192);
-      if (sp.sp > 1 && sp.full == 0) continue;
-    }
+    if (mc.cfg == kCfg192) continue;  // below
     const double us = model_us(M, N, K, mc);
     if (us < best_us) {
       best_us = us;
       best = mc.cfg;
     }
+  }
+  if (K % kRing192.bk == 0) {
+    const double us = model_us(M, N, K, kModel192);
+    if (us < best_us && ring192_pays(M, N, K, us, best, best_us)) best = kCfg192;
   }
   const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
   if (best == 2 && K % kStreamBK == 0 && K / kStreamBK >= kStreamMinStages && K / kStreamBK <= kStreamMaxStages &&

@@ -189,6 +189,20 @@ def test_few_walk_items_stay_on_the_tiles(lib):
         assert pref(*c) == 1, c
 
 
+def test_192_ring_only_where_it_pays(lib):
+    """The 192 x 256 ring leaves the shapes where it measured 4-30% slower
+    than its runner-up to that one, and keeps the ones it was made for
+    (choices for 256 CUs)."""
+    ring = b"tile3_gemm_kernel<192, 256, 128, 2, 4, 2>"
+    slower = [(301, 17408, 25600), (574, 12800, 17408), (435, 17408, 25600), (2131, 10240, 25600), (822, 17408, 17408),
+              (3428, 8192, 25600), (7475, 5120, 17408), (6403, 2048, 25600), (1629, 12240, 512), (800, 5120, 17408)]
+    for c in slower:
+        assert lib.mw8_gemm_kernel_name(*c) != ring, c
+    for c in [(2080, 5120, 25600), (2080, 5120, 17408), (2080, 5120, 8192), (2080, 10240, 5120), (2080, 51200, 5120),
+              (1500, 7168, 5120), (3000, 7168, 5120), (1024, 10240, 5120), (300, 34816, 5120), (566, 25600, 17408)]:
+        assert lib.mw8_gemm_kernel_name(*c) == ring, c
+
+
 def test_wrappers_load_on_a_cpu_only_torch():
     """A torch without GPU support lacks the bindings that name the current
     stream and device: the package still imports, and a wrapper refuses CPU

@@ -1,7 +1,7 @@
 """The 192 x 256 ring (tile configuration 13), forced: row counts around the
-tile height, ragged columns, one K stage to many, whole tiles and K splits of
-a short last wave, with and without bias, and with the gated activation in
-its epilogue.  Bit-exact against the oracle; the activation bit-identical to
+tile height, ragged columns, one K stage to many, whole tiles, K splits of
+every tile and of a short last wave behind whole tiles, with and without bias,
+and with the gated activation in its epilogue.  Bit-exact against the oracle; the activation bit-identical to
 the GEMM followed by the activation kernel."""
 
 import pytest
@@ -33,6 +33,25 @@ def forced():
 def test_forced(forced, M, N, K, bias):
     announce(f"192x256 M={M} N={N} K={K} bias={bias}")
     _run_case(M, K, N, seed=M + N + K, bias=bias)
+
+
+# tail tiles, K ranges of each: behind one whole wave of 256 tiles, by row tiles
+TAILS = [(300, 34816, 512, True, 16, 4), (100, 66000, 640, False, 2, 5), (3100, 4360, 768, True, 50, 5)]
+
+
+@pytest.mark.parametrize("M,N,K,bias,tail,ranges", TAILS)
+def test_split_last_wave(forced, M, N, K, bias, tail, ranges):
+    announce(f"192x256 split last wave M={M} N={N} K={K} bias={bias}")
+    assert -(-M // 192) * -(-N // 256) == 256 + tail
+    assert forced.mw8_gemm_workspace_bytes(M, N, K) == tail * ranges * 192 * 256 * 4
+    _run_case(M, K, N, seed=M + N, bias=bias)
+
+
+@pytest.mark.parametrize("M,I,K,act,tail,ranges", [(300, 17408, 512, "silu", 16, 4), (3100, 2184, 768, "gelu", 50, 5)])
+def test_activation_split_last_wave(forced, M, I, K, act, tail, ranges):
+    assert -(-M // 192) * -(-2 * I // 256) == 256 + tail
+    assert forced.mw8_gemm_act_workspace_bytes(M, I, K) == tail * ranges * 192 * 256 * 4
+    test_activation(forced, M, I, K, act)
 
 
 @pytest.mark.parametrize("M,I,K,act", [(192, 128, 128, "silu"), (200, 136, 512, "gelu"), (1000, 776, 1024, "silu"),
