@@ -105,11 +105,14 @@ def get_default_config(M: int, E: int, N: int, K: int, topk: int) -> Dict[str, i
     """Two tile regimes keyed on tokens vs experts, as the reference
     (python/minisgl/moe/fused.py:92-113), with the same keys.  BLOCK_SIZE_M
     is the alignment block: 16 rows when M <= E (decode: weight streaming),
-    otherwise 64 (MFMA tiles).  The other keys describe this build's
-    kernels for that regime: the weight rows a block streams and the K
-    bytes of one ring stage (16 rows x 256 bytes for 16-row blocks; 128 or
-    256 columns x 64 bytes for the tile walk), and GROUP_SIZE_M = 1 (the
-    tiles are ordered per XCD instead of by a GROUP_M swizzle)."""
+    otherwise 64 (MFMA tiles).  The other keys describe this build's basic
+    kernel for that regime: the weight rows a block streams and the K bytes
+    of one ring stage (16 rows x 256 bytes for 16-row blocks; 128 columns x
+    64 bytes for one tile per 64-row block), and GROUP_SIZE_M = 1 (the tiles
+    are ordered per XCD instead of by a GROUP_M swizzle).  The library
+    chooses the grouped GEMM over 64-row blocks from the sizes by itself: that
+    tile, a persistent walk with 128 x 256 tiles on 64-byte stages, or one
+    with 192 x 256 items on 128-byte stages."""
     if M <= E:
         return {"BLOCK_SIZE_M": 16, "BLOCK_SIZE_N": 16, "BLOCK_SIZE_K": 256, "GROUP_SIZE_M": 1}
     return {"BLOCK_SIZE_M": 64, "BLOCK_SIZE_N": 128, "BLOCK_SIZE_K": 64, "GROUP_SIZE_M": 1}

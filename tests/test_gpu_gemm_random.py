@@ -71,8 +71,9 @@ def test_gemm_random_wide_decode(M, N, K, bias):
 
 @pytest.mark.parametrize("M", [33, 64, 65, 127, 128, 192, 256])
 @pytest.mark.parametrize("N,K", [(5120, 5120), (7176, 4096)])
-def test_split_k_streamed_weights(M, N, K):
-    """The in-block split-K tiles at weights large enough to stream past the
-    L2s (20 MB and up), whole and ragged rows and columns."""
-    announce(f"streamed split-K M={M} N={N} K={K}")
+def test_split_k_tiles_model_sizes(M, N, K):
+    """The in-block split-K tiles at a model's weight sizes (26-29 MB), whole
+    and ragged rows and columns."""
+    announce(f"split-K M={M} N={N} K={K}")
+    assert load().mw8_gemm_kernel_name(M, N, K).startswith(b"ksplit_gemm_kernel<")
     _run_case(M, K, N, seed=M + N, bias=M % 2 == 1)
