@@ -74,6 +74,8 @@ def test_gemm_random_wide_decode(M, N, K, bias):
 def test_split_k_tiles_model_sizes(M, N, K):
     """The in-block split-K tiles at a model's weight sizes (26-29 MB), whole
     and ragged rows and columns."""
+    from minisgl_amd.kernel.lib import load
+
     announce(f"split-K M={M} N={N} K={K}")
     assert load().mw8_gemm_kernel_name(M, N, K).startswith(b"ksplit_gemm_kernel<")
     _run_case(M, K, N, seed=M + N, bias=M % 2 == 1)
