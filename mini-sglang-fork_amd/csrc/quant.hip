@@ -394,7 +394,7 @@ __global__ __launch_bounds__(TPR > 0 ? kBlock : 64 * kMaxWaves) void rmsnorm_row
 // 64 - 8192 rows and 65 - 4096 vectors: 1% off the fastest layout on average.
 enum class RowWork { kQuant, kAct, kNorm, kNormQuant };
 
-// Rows whose blocks of `waves` waves are resident at once.  A CU has 4 x 8
+// Rows whose blocks of `waves` waves are resident at once on `cus` CUs.  A CU has 4 x 8
 // wave slots, which blocks of a multiple of 4 waves fill; others pack worse
 // (10 waves: two blocks, not three; 5: some of the time five, counted only
 // if `loose`).  Blocks of one or two waves slow down before the slots are
@@ -404,21 +404,22 @@ enum class RowWork { kQuant, kAct, kNorm, kNormQuant };
 // 8; 420 x 20480 11.3 with 14 or 8, 12.3 with 10).
 inline bool heavy_rows(RowWork work) { return work == RowWork::kAct || work == RowWork::kNormQuant; }
 
-inline int64_t resident_rows(RowWork work, int64_t waves, bool loose) {
+inline int64_t resident_rows(RowWork work, int64_t cus, int64_t waves, bool loose) {
   if (waves > kMaxWaves) return 0;
   int64_t per_cu = waves % 4 == 0 || waves < 4 ? 32 / waves : 29 / waves;
   if (waves == 5 || waves == 6) per_cu = loose ? 5 : 4;
   if (waves >= 10 && heavy_rows(work)) per_cu = 1;
-  const int64_t rows = per_cu * device_cus();
+  const int64_t rows = per_cu * cus;
   return waves < 3 || (waves == 3 && work == RowWork::kNormQuant) ? rows * 3 / 4 : rows;
 }
 
 // The fewest vectors per thread, from `least` to `most`, of block rows whose
 // blocks are resident at once; 0: none.
 inline int resident_vectors(RowWork work, int64_t nvec, int64_t rows, int least, int most) {
+  const int64_t cus = device_cus();
   for (const bool loose : {false, true})
     for (int v = least; v <= most; ++v)
-      if (resident_rows(work, (nvec + 64 * v - 1) / (64 * v), loose) >= rows) return v;
+      if (resident_rows(work, cus, (nvec + 64 * v - 1) / (64 * v), loose) >= rows) return v;
   return 0;
 }
 
