@@ -3,15 +3,16 @@
 //
 // One block per CU (8 waves, 2 x 4 of 96 x 64) walks (expert, column tile,
 // row chunk) items of up to 192 sorted rows x 256 weight rows.  What bounds
-// it: at few rows per expert the weight stream from HBM (128 experts of 2048
-// x 1536: 403 MB in 67 us = 6.0 TB/s at 300 tokens), at 256 rows the stage
-// time of about 1.0 us, of which the MFMAs are 0.6, and the epilogue's VALU
-// work (about 4 us per item and SIMD for silu).
+// it (profiled at E 128, top-8, H 2048, I 768): at few rows per expert the
+// weight stream from HBM (300 tokens: GEMM1 reads 407 MB past L2, 403 of them
+// weights, in 69.9 us = 5.8 TB/s); at 256 rows a round of one item per CU, of
+// about 1.05 us per stage (its MFMAs 0.64 at the nominal rate) and 7.5 us
+// besides, in which the epilogue leaves the matrix cores idle (4096 tokens:
+// MFMA busy 0.32, a third of the wave cycles in waits).
 //
-//  * 128-byte row segments: the same operand stream in 64-byte segments
-//    reaches 8 TB/s through L2 against 11-13 (a stream of both operands into
-//    LDS without MFMAs), and was the bound of the 128 x 256 tiles on 64-byte
-//    stages that this walk replaces (4096 tokens: 1.4 GB in 180 us).
+//  * 128-byte row segments: 1.33 GB of operands move through L2 in 146 us
+//    (GEMM1, 4096 tokens, 9.2 TB/s), where the 128 x 256 tiles on 64-byte
+//    stages that this walk replaces took 186 us.
 //  * The two operands have rings and loading waves of their own: waves 0-3
 //    load A (2 slots of 24 KB: the gathered rows mostly hit in L2), waves
 //    4-7 W (3 slots of 32 KB: the weights come from HBM, about 1.5 us away).
@@ -22,8 +23,7 @@
 //    not queue in front of the A loads (4096 tokens: 173 -> 159 us).
 //  * Weights stream with the non-temporal policy, also where two chunks
 //    share them (side by side on one XCD): they would evict the rows that
-//    the expert's other column tiles re-read (operand stream alone: 118 ->
-//    97 us with two chunks).
+//    the expert's other column tiles re-read.
 //  * The rings run on across items: the next item's first stages are issued
 //    during the current item's last ones and land while it writes its
 //    output.
@@ -33,7 +33,7 @@
 //    v_permlane16_swap per packed word makes them 16-byte row segments, and
 //    each wave stores its own columns.  No LDS staging, no barrier, and the
 //    ring keeps its slots.
-//  * 16-row fragments past an expert's rows skip their MFMAs (one instance
+//  * 16-row fragments past a chunk's last pair skip their MFMAs (one instance
 //    of the stage loop per count, no branch inside); the fragments of a
 //    chunk are dealt to the two wave rows in turn, so a short chunk stays
 //    balanced; rows past them read zeros without traffic.
