@@ -7,7 +7,7 @@
 //
 // One row is owned by TPR threads: 16 or 32 (part of a wave, several rows
 // per wave), 64 (a wave, four rows per block), or 0 = the whole block, one
-// row per block of 128 - 1024 threads.  Each thread keeps VPT 16-byte
+// row per block of 64 - 1024 threads.  Each thread keeps VPT 16-byte
 // vectors (8 bf16) of the row in registers, so the row is read from HBM
 // once: 16-byte coalesced loads, an integer max over the sign-cleared bf16
 // bit patterns (monotone for finite values), a wave/LDS max-reduction, then
