@@ -383,12 +383,12 @@ __global__ __launch_bounds__(TPR > 0 ? kBlock : 64 * kMaxWaves) void rmsnorm_row
 // 5; 3, 4, 6, 7 80.4, 77.4, 77.0, 79.0).  The activation and the quantizing
 // norm compute more per vector and want more threads: from 193 to 1024
 // vectors 2 per thread (norm + residual 8192 x 4096 51.8 us on a wave per row
-// -> 43.6, 8192 x 5120 53.6 with 3 -> 52.8), residency with at most 5 and 4,
+// -> 43.6, 8192 x 5120 53.7 with 3 -> 52.5), residency with at most 5 and 4,
 // and past 768 vectors (12 waves) the norm never 1 (1 x 8192 5.2 us, with 2
 // 4.8; 1 x 6144 4.4 and 4.6).
 // Rows of 65 - 128 vectors: blocks up to 3072 rows (plain norm 2304, with the
 // quantizer 1024), then wave rows, two to a wave up to 96 vectors (act 8192 x
-// 768 9.7 us on one -> 8.9; the norms from 4096 rows).
+// 768 9.8 us on one -> 8.9; the norms from 4096 rows).
 //
 // MI355X, graph nodes of 10 rotating inputs, 1436 combinations of operation,
 // 64 - 8192 rows and 65 - 4096 vectors: 1% off the fastest layout on average.
